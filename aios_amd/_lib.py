@@ -35,6 +35,7 @@ EXPORTED_SYMBOLS = (
     "aios_kv_append",
     "aios_attn_plan",
     "aios_attn_prefill",
+    "aios_attn_prefill_ws",
     "aios_attn_decode",
     "aios_attn_append_decode",
     "aios_attn_append_decode_rope",
@@ -119,6 +120,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.aios_attn_prefill.restype = ctypes.c_int
     lib.aios_attn_prefill.argtypes = [
         ctypes.POINTER(AttnPlan), _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _f32, _vp,
+    ]
+    lib.aios_attn_prefill_ws.restype = ctypes.c_int
+    lib.aios_attn_prefill_ws.argtypes = [
+        ctypes.POINTER(AttnPlan), _vp, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _f32,
+        _vp,
     ]
     lib.aios_attn_decode.restype = ctypes.c_int
     lib.aios_attn_decode.argtypes = [

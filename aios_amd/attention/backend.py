@@ -295,7 +295,7 @@ class Mi355xAttentionBackend(BaseAttentionBackend):
             shared_prefix_len=shared,
             host_staging=host,
         )
-        if plan.ws_bytes:
+        if plan.ws_bytes and batch.is_decode:
             self._get_workspace(device)
         batch.attn_metadata = metadata
         return metadata

@@ -1,4 +1,5 @@
 // C ABI of the attention backend: validation, host-side planning and launch.
+#include <math.h>
 #include <stdarg.h>
 #include <stdlib.h>
 #include <stdio.h>
@@ -32,6 +33,24 @@ int32_t cdiv(int32_t a, int32_t b) { return (a + b - 1) / b; }
 
 // Shared prefixes shorter than this are read per row (no second launch).
 constexpr int32_t kMinCascadePrefix = 256;
+// Prefill split, in 32-position sub-tiles (measured on MI355X with both sides
+// of each line; per layer, main launch + combine against one workgroup per
+// tile).
+// Few-row tiles (at most 64 MFMA rows) longer than 6 sub-tiles: 8 tokens of a
+// 32q/8kv x 128 model against 188 positions 8.7 us unsplit and 10.0 split,
+// against 258 positions 11.1 and 10.0, 6 against 4,099 94.7 and 16.2.
+constexpr int32_t kPrefillFewUnsplit = 6;
+// Fuller tiles: a part costs about 8 sub-tiles' time (launch, state, merge)
+// and the last part half its length, so a part of 4 sqrt(work per compute
+// unit) sub-tiles balances the two (100 tokens against 4,100 positions: 102
+// us unsplit; parts of 4 / 8 / 12 / 16 / 24 sub-tiles 40 / 32 / 28 / 28 / 32
+// us); at most about two parts per compute unit, which are all resident at
+// once (a 2,048-token prompt, 16q/8kv x 128: 57 us; 12 / 16 / 24 / 32: 58 /
+// 50 / 42 / 46 us).  From 7/4 tiles per compute unit on the causal tiles fill
+// the chip by themselves (4,096 tokens, 16q/8kv: 114 us unsplit, 107 at best).
+constexpr int32_t kPrefillMinSplit = 16;  // shorter tiles: 300 tokens 13.8 us, split 15.5-16.3
+constexpr int32_t kPrefillMinPart = 6;
+constexpr int32_t kPrefillMinGain = 11;   // sub-tiles off the longest workgroup
 // Partial states per (row, kv-head) the combine merges (one per lane of a
 // wavefront when it computes the merge weights).
 constexpr int32_t kMaxParts = 64;
@@ -50,6 +69,62 @@ int device_cus() {
       cus = 256;
   }
   return cus;
+}
+
+// How a prefill batch splits its tiles' KV ranges over workgroups
+// (prefix_chunk_len: positions per part, 0 = unsplit; num_parts: most parts
+// of a tile).  Work is counted in 32-position sub-tiles of a (tile, kv-head).
+void plan_prefill_parts(aios_attn_plan_t* p, const int32_t* cu_q, const int32_t* cu_k, int32_t cus,
+                        int64_t ws_bytes) {
+  const int32_t G = p->group, q_tile = p->prefill_q_tile, hkv = p->num_kv_heads;
+  const int32_t rows = (p->max_q_len < q_tile ? p->max_q_len : q_tile) * G;
+  auto each_tile = [&](auto&& f) {
+    for (int32_t b = 0; b < p->batch_size; ++b) {
+      const int32_t ql = cu_q[b + 1] - cu_q[b];
+      const int32_t kl = cu_k[b + 1] - cu_k[b];
+      for (int32_t q0 = 0; q0 < ql; q0 += q_tile)
+        f(cdiv(kl - ql + (q0 + q_tile < ql ? q0 + q_tile : ql), 32));
+    }
+  };
+  int64_t work = 0, tiles = 0;
+  int32_t longest = 0;
+  each_tile([&](int32_t sub) {
+    work += (int64_t)sub * hkv;
+    tiles += hkv;
+    if (sub > longest) longest = sub;
+  });
+  auto count_parts = [&](int32_t part_sub) {
+    int64_t n = 0;
+    each_tile([&](int32_t sub) { n += (int64_t)cdiv(sub, part_sub) * hkv; });
+    return n;
+  };
+  int32_t part_sub;
+  if (rows <= 64) {
+    if (longest <= kPrefillFewUnsplit) return;
+    part_sub = aios::kPrefillFewSub;
+  } else {
+    if (longest < kPrefillMinSplit || 4 * tiles >= 7 * cus) return;
+    part_sub = (int32_t)(4.0 * sqrt((double)work / cus) + 0.5);
+    if (part_sub < kPrefillMinPart) part_sub = kPrefillMinPart;
+    while (2 * part_sub <= 3 * longest &&
+           (100 * work > 97 * 2ll * cus * cdiv(longest, cdiv(longest, part_sub)) ||
+            3 * count_parts(part_sub) > 7 * cus))
+      part_sub += 1 + part_sub / 16;
+    const int32_t gain = longest - part_sub;
+    if (gain < kPrefillMinGain || 2 * gain < part_sub) return;
+  }
+  const int32_t n = cdiv(longest, part_sub);
+  const int64_t parts = (int64_t)p->batch_size * p->num_q_tiles * hkv * n;
+  const int64_t o_bytes = parts * aios::kPrefillRows * p->head_dim * 4;
+  const int64_t bytes = n > 1 ? o_bytes + align_up(parts * aios::kPrefillRows * 8, 256) : 0;
+  if (bytes > ws_bytes || parts > 0x3fffffff) return;
+  p->prefix_chunk_len = part_sub * 32;
+  p->num_parts = n;
+  if (n > 1) {
+    p->ws_parts_o = 0;
+    p->ws_parts_lse = o_bytes;
+    p->ws_bytes = bytes;
+  }
 }
 
 }  // namespace
@@ -129,6 +204,7 @@ int aios_attn_plan(int32_t phase, const int32_t* cu_q, const int32_t* cu_k, int3
     const int32_t q_tile = 128 / G;
     p->prefill_q_tile = q_tile;
     p->num_q_tiles = max_q > 0 ? cdiv(max_q, q_tile) : 0;
+    plan_prefill_parts(p, cu_q, cu_k, cus, ws_bytes);
     return AIOS_OK;
   }
 
@@ -237,6 +313,15 @@ int aios_attn_prefill(const aios_attn_plan_t* p, const void* q, int64_t q_tok_st
                       const void* k_cache, const void* v_cache, int64_t kv_num_pages,
                       const int32_t* indices, const int32_t* cu_q, const int32_t* cu_k, void* out,
                       float sm_scale, void* stream) {
+  return aios_attn_prefill_ws(p, q, q_tok_stride, k_cache, v_cache, kv_num_pages, indices, cu_q,
+                              cu_k, out, nullptr, 0, sm_scale, stream);
+}
+
+int aios_attn_prefill_ws(const aios_attn_plan_t* p, const void* q, int64_t q_tok_stride,
+                         const void* k_cache, const void* v_cache, int64_t kv_num_pages,
+                         const int32_t* indices, const int32_t* cu_q, const int32_t* cu_k,
+                         void* out, void* workspace, int64_t workspace_bytes, float sm_scale,
+                         void* stream) {
   int rc = check_plan(p, AIOS_PHASE_PREFILL);
   if (rc) return rc;
   if (p->batch_size == 0 || p->total_q == 0) return AIOS_OK;
@@ -267,6 +352,21 @@ int aios_attn_prefill(const aios_attn_plan_t* p, const void* q, int64_t q_tok_st
   a.q_tiles = p->num_q_tiles;
   a.batch = p->batch_size;
   a.out = static_cast<aios::bf16*>(out);
+  // Split tiles need room for their partial states; without it (or with a
+  // plan that has none) each tile is one workgroup.
+  if (p->num_parts > 0 && (p->ws_bytes == 0 || (workspace && p->ws_bytes <= workspace_bytes))) {
+    if (((uintptr_t)workspace & 255) != 0)
+      return fail(AIOS_ERR_INVALID, "prefill: workspace must be 256-byte aligned");
+    char* ws = static_cast<char*>(workspace);
+    a.part_sub = p->prefix_chunk_len / 32;
+    a.n_parts = p->num_parts;
+    a.part_o = reinterpret_cast<float*>(ws + p->ws_parts_o);
+    a.part_ml = reinterpret_cast<float2*>(ws + p->ws_parts_lse);
+    const int32_t tok = p->max_q_len < a.q_tile ? p->max_q_len : a.q_tile;
+    return check_hip(aios::launch_prefill_split(D, a, tok * a.group,
+                                                static_cast<hipStream_t>(stream)),
+                     "prefill launch");
+  }
   return check_hip(aios::launch_prefill(D, 4, a, p->num_q_tiles, p->batch_size,
                                         static_cast<hipStream_t>(stream)),
                    "prefill launch");

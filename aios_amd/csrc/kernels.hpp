@@ -102,7 +102,37 @@ struct PrefillArgs {
   int32_t q_tiles;  // query tiles of the longest request
   int32_t batch;
   bf16* out;
+  // Split of each tile's KV range over several workgroups (part_sub > 0):
+  // parts of about part_sub 32-position sub-tiles, at most n_parts a tile.
+  // The partial states of tile slot t = (r * q_tiles + qt) * Hkv + h, part s
+  // (s < the tile's own part count), all fp32 and relative to the row's
+  // reference m:
+  //   part_o  [slots][n_parts][D / 8][kPrefillRows][8]  unnormalised o
+  //   part_ml [slots][n_parts][kPrefillRows]            (m, row sum l)
+  // A tile of one part writes bf16 output directly.
+  int32_t part_sub;
+  int32_t n_parts;
+  float* part_o;
+  float2* part_ml;
 };
+
+constexpr int kPrefillRows = 128;  // MFMA rows of a prefill query tile
+constexpr int kPrefillFewSub = 4;  // sub-tiles of a few-row tile's part: the LDS ring
+
+// The parts of a tile whose KV range holds kv positions: n of them, per
+// sub-tiles each (the last one may be shorter).
+struct PrefillParts {
+  int32_t n, per;
+};
+__host__ __device__ inline PrefillParts prefill_parts(int32_t kv, int32_t part_sub,
+                                                      int32_t n_parts) {
+  const int32_t n_sub = (kv + 31) / 32;
+  int32_t n = (n_sub + part_sub - 1) / part_sub;
+  n = n < n_parts ? n : n_parts;
+  if (n < 1) n = 1;
+  const int32_t per = n_sub > n ? (n_sub + n - 1) / n : 1;
+  return PrefillParts{(n_sub + per - 1) / per, per};
+}
 
 hipError_t kv_append(void* k_cache, void* v_cache, int64_t num_slots, int64_t cache_stride_b,
                      const int32_t* out_loc, const void* k, int64_t k_stride_b, const void* v,
@@ -251,6 +281,9 @@ hipError_t launch_decode_combine(int D, const DecodeArgs& a, hipStream_t stream)
 
 hipError_t launch_prefill(int D, int NW, const PrefillArgs& a, int q_tiles, int batch,
                           hipStream_t stream);
+// The same with each tile's KV range split (a.part_sub > 0): rows_max = MFMA
+// rows of the fullest tile.
+hipError_t launch_prefill_split(int D, const PrefillArgs& a, int rows_max, hipStream_t stream);
 
 bool head_dim_supported(int D);
 bool group_supported(int G);

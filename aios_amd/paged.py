@@ -235,13 +235,16 @@ def prefill(p: _lib.AttnPlan, q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
     if out is None:
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     scale = p.head_dim ** -0.5 if sm_scale is None else sm_scale
+    # The partial states of a split batch live in a buffer of this call alone
+    # (from torch's allocator, on the current stream): prefills of one plan or
+    # backend may run on several streams and threads.
+    ws = torch.empty(p.ws_bytes, dtype=torch.uint8, device=q.device) if p.ws_bytes else None
     _lib.check(
-        _lib.lib().aios_attn_prefill(
+        _lib.lib().aios_attn_prefill_ws(
             p, q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
             k_cache.shape[0], indices.data_ptr(), cu_q.data_ptr(), cu_k.data_ptr(), out.data_ptr(),
-            scale,
-            _stream(q.device)),
-        "aios_attn_prefill",
+            ws.data_ptr() if ws is not None else None, p.ws_bytes, scale, _stream(q.device)),
+        "aios_attn_prefill_ws",
     )
     return out
 

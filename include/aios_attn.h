@@ -118,6 +118,9 @@ typedef struct aios_attn_plan {
   /* prefill */
   int32_t prefill_q_tile;    /* query tokens per workgroup */
   int32_t num_q_tiles;
+  /* (a prefill whose KV ranges are split over workgroups also sets
+   * prefix_chunk_len, the KV positions per part, num_parts, the most parts
+   * of a tile, and the workspace fields) */
   /* decode launches to issue: bit 0 the main kernel (prefix chunks and
    * suffix items), bit 1 the combine; 0 (the value aios_attn_plan writes)
    * issues both.  Lets a profiler bracket the two launches separately. */
@@ -170,6 +173,21 @@ int aios_attn_prefill(const aios_attn_plan_t* plan, const void* q,
                       const int32_t* indices,
                       const int32_t* cu_q, const int32_t* cu_k, void* out,
                       float sm_scale, void* stream);
+
+/*
+ * aios_attn_prefill with a workspace for the partial softmax states (fp32) of
+ * batches with too few query tiles to fill the GPU: each tile's KV range is
+ * then split over several workgroups and merged by a second launch.  Used
+ * when workspace is given, 256-byte aligned, and holds plan->ws_bytes;
+ * otherwise, as aios_attn_prefill, every tile is one workgroup.
+ */
+int aios_attn_prefill_ws(const aios_attn_plan_t* plan, const void* q,
+                         int64_t q_tok_stride, const void* k_cache,
+                         const void* v_cache, int64_t kv_num_pages,
+                         const int32_t* indices,
+                         const int32_t* cu_q, const int32_t* cu_k, void* out,
+                         void* workspace, int64_t workspace_bytes,
+                         float sm_scale, void* stream);
 
 /*
  * Paged decode (kernels (c) + (d) + log-sum-exp combine), bf16.  Row b has

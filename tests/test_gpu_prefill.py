@@ -121,3 +121,44 @@ def test_growing_logits_move_the_softmax_reference(q_lens, kv_lens, hq, hkv, d):
     kc = (kc.float() * scale.view(-1, 1, 1)).to(torch.bfloat16)
     out, _ = _run(q, kc, vc, idx, cu_q, cu_k, hq, hkv, d)
     np.testing.assert_allclose(to_np64(out), _oracle(q, kc, vc, idx, cu_q, cu_k, d), **BF16_TOL)
+
+
+@pytest.mark.parametrize("q_lens,kv_lens,hq,hkv,d", [
+    ([1], [193], 8, 8, 64),                    # few rows: the shortest split range, one row
+    ([8], [513], 32, 8, 128),                  # one full 32-row tile, one position over a part
+    ([9], [1000], 32, 8, 128),                 # 36 rows: two row tiles, half the wavefronts each
+    ([16, 1, 3], [900, 300, 40], 8, 2, 96),    # ragged few-row batch, one tile unsplit
+    ([21], [2100], 12, 4, 64),                 # G = 3: 63 rows
+    ([10], [700], 48, 8, 64),                  # G = 6
+    ([65], [1400], 16, 8, 128),                # fuller tiles (ring path), a second short tile
+    ([150, 33], [1500, 1033], 8, 2, 96),
+    ([300], [1300], 12, 4, 64),
+])
+def test_split_kv_ranges_match_oracle(q_lens, kv_lens, hq, hkv, d):
+    # Batches whose tiles' KV ranges are split over workgroups; K rows grow
+    # along the positions, so the parts' softmax references differ widely.
+    q, kc, vc, idx, cu_q, cu_k = _make(q_lens, kv_lens, hq, hkv, d, 4096, seed=sum(kv_lens))
+    scale = torch.ones(kc.shape[0])
+    for r in range(len(kv_lens)):
+        lo, hi = int(cu_k[r]), int(cu_k[r + 1])
+        scale[idx[lo:hi].long()] = 1.0 + 20.0 * torch.arange(hi - lo, dtype=torch.float32) / (hi - lo)
+    kc = (kc.float() * scale.view(-1, 1, 1)).to(torch.bfloat16)
+    out, p = _run(q, kc, vc, idx, cu_q, cu_k, hq, hkv, d)
+    assert p.num_parts > 1 and p.ws_bytes > 0
+    ref = _oracle(q, kc, vc, idx, cu_q, cu_k, d)
+    np.testing.assert_allclose(to_np64(out), ref, **BF16_TOL)
+    # a plan for longer ranges (a replayed prefill's capacity) on the same batch
+    cap = cu_k.clone()
+    cap[1:] += 320 * torch.arange(1, len(cap), dtype=torch.int32)
+    wide = paged.plan("prefill", cu_q, cap, hq, hkv, d)
+    roomy = torch.zeros(int(cap[-1]), dtype=torch.int32)
+    roomy[: idx.numel()] = idx
+    out = paged.prefill(wide, q.to(DEV), kc.to(DEV), vc.to(DEV), roomy.to(DEV), cu_q.to(DEV),
+                        cu_k.to(DEV))
+    np.testing.assert_allclose(to_np64(out), ref, **BF16_TOL)
+    # a plan without room for the states keeps one workgroup per tile
+    small = paged.plan("prefill", cu_q, cu_k, hq, hkv, d, workspace_bytes=1024)
+    assert small.num_parts == 0 and small.ws_bytes == 0
+    out = paged.prefill(small, q.to(DEV), kc.to(DEV), vc.to(DEV), idx.to(DEV), cu_q.to(DEV),
+                        cu_k.to(DEV))
+    np.testing.assert_allclose(to_np64(out), ref, **BF16_TOL)
