@@ -42,6 +42,7 @@ EXPORTED_SYMBOLS = (
     "aios_attn_decode_noalloc",
     "aios_build_indices",
     "aios_rmsnorm",
+    "aios_add_rmsnorm",
     "aios_qk_norm_rope",
     "aios_cg_step_begin",
     "aios_cg_step_end",
@@ -49,6 +50,8 @@ EXPORTED_SYMBOLS = (
     "aios_silu_mul",
     "aios_linear_rows",
     "aios_linear_rows_ex",
+    "aios_linear_rows_workspace",
+    "aios_linear_rows_ws",
     "aios_greedy_select",
     "aios_attnres_mix",
     "aios_attnres_mix_ex",
@@ -146,6 +149,9 @@ def _declare(lib: ctypes.CDLL) -> None:
     ]
     lib.aios_build_indices.restype = ctypes.c_int
     lib.aios_build_indices.argtypes = [_vp, _i64, _vp, _vp, _i32, _i32, _vp, _vp]
+    lib.aios_add_rmsnorm.restype = ctypes.c_int
+    lib.aios_add_rmsnorm.argtypes = [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _i64, _i64, _i32,
+                                     _f32, _vp]
     lib.aios_rmsnorm.restype = ctypes.c_int
     lib.aios_rmsnorm.argtypes = [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i32, _f32, _vp]
     lib.aios_cg_step_begin.restype = ctypes.c_int
@@ -163,6 +169,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.aios_silu_mul.argtypes = [_vp, _i64, _i64, _i32, _vp, _i64, _vp]
     lib.aios_linear_rows.restype = ctypes.c_int
     lib.aios_linear_rows.argtypes = [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp]
+    lib.aios_linear_rows_workspace.restype = _i64
+    lib.aios_linear_rows_workspace.argtypes = [_i64, _i64, _i64]
+    lib.aios_linear_rows_ws.restype = ctypes.c_int
+    lib.aios_linear_rows_ws.argtypes = [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i32,
+                                        _vp, _i64, _vp, _f32, _vp, _i64, _i32, _vp, _i64, _vp]
     lib.aios_linear_rows_ex.restype = ctypes.c_int
     lib.aios_linear_rows_ex.argtypes = [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i32,
                                         _vp, _i64, _vp, _f32, _vp, _i64, _i32, _vp]

@@ -71,6 +71,14 @@ int device_cus() {
   return cus;
 }
 
+// Projections that take the streaming form (gemm_rows.hip): more rows than one
+// 16-row tile, or a K without a fixed-K instance in gemm_skinny.hip, which
+// are the faster ones where they exist (8 rows, N x K 4096 x 1024: 3.9 us
+// against 5.0; 1024 x 2048: 4.4 against 6.0).
+bool rows_form(int64_t rows, int64_t k, bool norm) {
+  return rows > 16 || (k > 1024 && (norm || (k != 2048 && k != 3072)));
+}
+
 // How a prefill batch splits its tiles' KV ranges over workgroups
 // (prefix_chunk_len: positions per part, 0 = unsplit; num_parts: most parts
 // of a tile).  Work is counted in 32-position sub-tiles of a (tile, kv-head).
@@ -630,9 +638,31 @@ int aios_rmsnorm(const void* x, int64_t x_stride, void* residual, int64_t residu
     return fail(AIOS_ERR_INVALID, "rmsnorm: row strides must be >= hidden and multiples of 8");
   if ((((uintptr_t)x | (uintptr_t)weight | (uintptr_t)out | (uintptr_t)residual) & 15) != 0)
     return fail(AIOS_ERR_INVALID, "rmsnorm: rows must be 16-byte aligned");
-  return check_hip(aios::rmsnorm(x, x_stride, residual, residual_stride, weight, out, out_stride,
-                                 rows, hidden, eps, static_cast<hipStream_t>(stream)),
+  return check_hip(aios::rmsnorm(x, x_stride, residual, residual_stride, residual, residual_stride,
+                                 weight, out, out_stride, rows, hidden, eps,
+                                 static_cast<hipStream_t>(stream)),
                    "rmsnorm launch");
+}
+
+int aios_add_rmsnorm(const void* x, int64_t x_stride, const void* residual, int64_t residual_stride,
+                     const void* weight, void* residual_out, int64_t residual_out_stride, void* out,
+                     int64_t out_stride, int64_t rows, int32_t hidden, float eps, void* stream) {
+  if (rows < 0 || !aios::rmsnorm_supported(hidden))
+    return fail(AIOS_ERR_INVALID, "add_rmsnorm: hidden %d must be a multiple of 8 up to 8192", hidden);
+  if (rows == 0) return AIOS_OK;
+  if (!x || !residual || !weight || !residual_out || !out)
+    return fail(AIOS_ERR_INVALID, "add_rmsnorm: null pointer");
+  if (x_stride < hidden || out_stride < hidden || residual_stride < hidden ||
+      residual_out_stride < hidden ||
+      (x_stride | out_stride | residual_stride | residual_out_stride) % 8 != 0)
+    return fail(AIOS_ERR_INVALID, "add_rmsnorm: row strides must be >= hidden and multiples of 8");
+  if ((((uintptr_t)x | (uintptr_t)weight | (uintptr_t)out | (uintptr_t)residual |
+        (uintptr_t)residual_out) & 15) != 0)
+    return fail(AIOS_ERR_INVALID, "add_rmsnorm: rows must be 16-byte aligned");
+  return check_hip(aios::rmsnorm(x, x_stride, residual, residual_stride, residual_out,
+                                 residual_out_stride, weight, out, out_stride, rows, hidden, eps,
+                                 static_cast<hipStream_t>(stream)),
+                   "add_rmsnorm launch");
 }
 
 int aios_qk_norm_rope(const void* qkv, int64_t qkv_stride, int64_t tokens, int32_t num_qo_heads,
@@ -689,6 +719,31 @@ int aios_linear_rows_ex(const void* x, int64_t x_stride, const void* weight, int
                         int64_t residual_stride, const void* norm_weight, float eps,
                         void* residual_out, int64_t residual_out_stride, int32_t epilogue,
                         void* stream) {
+  if (prologue == AIOS_PROLOGUE_ADD_RMSNORM &&
+      aios::skinny_gemm_supported(rows, out_features, in_features) &&
+      !aios::skinny_gemm_norm_supported(rows, in_features))
+    return fail(AIOS_ERR_UNSUPPORTED, "linear_rows: RMSNorm prologue for %lld rows x %lld",
+                (long long)rows, (long long)in_features);
+  return aios_linear_rows_ws(x, x_stride, weight, w_stride, y, y_stride, rows, out_features,
+                             in_features, prologue, residual, residual_stride, norm_weight, eps,
+                             residual_out, residual_out_stride, epilogue, nullptr, 0, stream);
+}
+
+int64_t aios_linear_rows_workspace(int64_t rows, int64_t out_features, int64_t in_features) {
+  aios::RowsPlan p;
+  if (!aios::skinny_gemm_supported(rows, out_features, in_features) ||
+      !rows_form(rows, in_features, false) ||
+      !aios::rows_gemm_plan(rows, out_features, in_features, false, false, true, device_cus(), &p))
+    return 0;
+  return p.bytes;
+}
+
+int aios_linear_rows_ws(const void* x, int64_t x_stride, const void* weight, int64_t w_stride,
+                        void* y, int64_t y_stride, int64_t rows, int64_t out_features,
+                        int64_t in_features, int32_t prologue, const void* residual,
+                        int64_t residual_stride, const void* norm_weight, float eps,
+                        void* residual_out, int64_t residual_out_stride, int32_t epilogue,
+                        void* workspace, int64_t workspace_bytes, void* stream) {
   if (!aios::skinny_gemm_supported(rows, out_features, in_features))
     return fail(AIOS_ERR_UNSUPPORTED,
                 "linear_rows: needs 1..64 rows, out_features %% 16 == 0, in_features %% 128 == 0 "
@@ -698,9 +753,6 @@ int aios_linear_rows_ex(const void* x, int64_t x_stride, const void* weight, int
     return fail(AIOS_ERR_INVALID, "linear_rows: unknown prologue %d", prologue);
   if (epilogue != AIOS_EPILOGUE_NONE && epilogue != AIOS_EPILOGUE_SILU_MUL)
     return fail(AIOS_ERR_INVALID, "linear_rows: unknown epilogue %d", epilogue);
-  if (prologue == AIOS_PROLOGUE_ADD_RMSNORM && !aios::skinny_gemm_norm_supported(rows, in_features))
-    return fail(AIOS_ERR_UNSUPPORTED, "linear_rows: RMSNorm prologue for %lld rows x %lld",
-                (long long)rows, (long long)in_features);
   if (!x || !weight || !y) return fail(AIOS_ERR_INVALID, "linear_rows: null pointer");
   if (x_stride < in_features || w_stride < in_features || y_stride < out_features ||
       (x_stride | w_stride) % 8 != 0 || y_stride % 4 != 0)
@@ -735,6 +787,22 @@ int aios_linear_rows_ex(const void* x, int64_t x_stride, const void* weight, int
   a.eps = eps;
   a.residual_out = static_cast<aios::bf16*>(residual_out);
   a.ro_stride = residual_out_stride;
+  const bool norm = prologue == AIOS_PROLOGUE_ADD_RMSNORM;
+  const bool silu = epilogue == AIOS_EPILOGUE_SILU_MUL;
+  if (rows_form(rows, in_features, norm) && aios::rows_gemm_fits(a, silu)) {
+    const bool ws = workspace && ((uintptr_t)workspace & 15) == 0;
+    aios::RowsPlan p;
+    bool ok = aios::rows_gemm_plan(rows, out_features, in_features, norm, silu, ws, device_cus(), &p);
+    if (ok && p.bytes > workspace_bytes)
+      ok = aios::rows_gemm_plan(rows, out_features, in_features, norm, silu, false, device_cus(), &p);
+    if (ok)
+      return check_hip(aios::rows_gemm(a, norm, silu, p, workspace,
+                                       static_cast<hipStream_t>(stream)),
+                       "linear_rows launch");
+  }
+  if (norm && !aios::skinny_gemm_norm_supported(rows, in_features))
+    return fail(AIOS_ERR_UNSUPPORTED, "linear_rows: RMSNorm prologue for %lld rows x %lld",
+                (long long)rows, (long long)in_features);
   return check_hip(aios::skinny_gemm(a, prologue, epilogue, static_cast<hipStream_t>(stream)),
                    "linear_rows launch");
 }

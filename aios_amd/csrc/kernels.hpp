@@ -143,9 +143,9 @@ hipError_t build_indices(const int32_t* page_table, int64_t pt_stride, const int
                          const int32_t* cu_k, int32_t batch, int32_t max_len,
                          int32_t* indices, hipStream_t stream);
 
-hipError_t rmsnorm(const void* x, int64_t x_stride, void* residual, int64_t r_stride,
-                   const void* w, void* out, int64_t out_stride, int64_t rows, int hidden,
-                   float eps, hipStream_t stream);
+hipError_t rmsnorm(const void* x, int64_t x_stride, const void* residual, int64_t r_stride,
+                   void* residual_out, int64_t ro_stride, const void* w, void* out,
+                   int64_t out_stride, int64_t rows, int hidden, float eps, hipStream_t stream);
 bool rmsnorm_supported(int hidden);
 
 hipError_t qk_norm_rope(const void* qkv, int64_t stride, int64_t tokens, int hq, int hkv, int D,
@@ -215,6 +215,18 @@ hipError_t cg_step_end(const CgStepArgs& a, hipStream_t stream);
 bool skinny_gemm_supported(int64_t M, int64_t N, int64_t K);
 bool skinny_gemm_norm_supported(int64_t M, int64_t K);
 hipError_t skinny_gemm(const LinearArgs& a, int prologue, int epilogue, hipStream_t stream);
+
+// The streaming form (gemm_rows.hip): K over `splits` groups of workgroups, ks
+// register steps per wavefront, bytes of fp32 partial products.
+struct RowsPlan {
+  int32_t splits, ks, grid;
+  int64_t bytes;
+};
+bool rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool norm, bool silu, bool workspace, int cus,
+                    RowsPlan* plan);
+bool rows_gemm_fits(const LinearArgs& a, bool silu);
+hipError_t rows_gemm(const LinearArgs& a, bool norm, bool silu, const RowsPlan& p, void* workspace,
+                     hipStream_t stream);
 
 hipError_t greedy_select(const void* logits, int64_t row_stride, int32_t rows, int32_t vocab,
                          int32_t elem_bytes, int64_t* token_out, float* logprob_out,

@@ -39,15 +39,17 @@ __device__ __forceinline__ uint4 pack8(const float* f) {
 }
 
 // One workgroup per row.  residual == nullptr: out = rmsnorm(x) * w.
-// Otherwise r = x + residual (fp32), residual <- bf16(r), out = rmsnorm(r) * w.
-// out may alias x: each thread writes only the elements it read.
+// Otherwise r = x + residual (fp32), residual_out <- bf16(r), out = rmsnorm(r) * w.
+// out may alias x, and residual_out residual: each thread writes only the
+// elements it read.
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(
-    const bf16* x, int64_t x_stride, bf16* residual, int64_t r_stride,
-    const bf16* __restrict__ w, bf16* out, int64_t out_stride, int hidden, float eps) {
+    const bf16* x, int64_t x_stride, const bf16* residual, int64_t r_stride, bf16* residual_out,
+    int64_t ro_stride, const bf16* __restrict__ w, bf16* out, int64_t out_stride, int hidden, float eps) {
   __shared__ float red[kNormThreads / 64];
   const int64_t row = blockIdx.x;
   const bf16* xr = x + row * x_stride;
-  bf16* rr = residual ? residual + row * r_stride : nullptr;
+  const bf16* rr = residual ? residual + row * r_stride : nullptr;
+  bf16* ro = residual ? residual_out + row * ro_stride : nullptr;
   float v[kNormMaxVec][8];
   float ss = 0.f;
 #pragma unroll
@@ -60,7 +62,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(
         unpack8(*reinterpret_cast<const uint4*>(rr + i), r);
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[k][j] += r[j];
-        *reinterpret_cast<uint4*>(rr + i) = pack8(v[k]);
+        *reinterpret_cast<uint4*>(ro + i) = pack8(v[k]);
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss = fmaf(v[k][j], v[k][j], ss);
@@ -159,12 +161,13 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const bf16* __restrict__ 
 
 }  // namespace
 
-hipError_t rmsnorm(const void* x, int64_t x_stride, void* residual, int64_t r_stride,
-                   const void* w, void* out, int64_t out_stride, int64_t rows, int hidden,
-                   float eps, hipStream_t stream) {
+hipError_t rmsnorm(const void* x, int64_t x_stride, const void* residual, int64_t r_stride,
+                   void* residual_out, int64_t ro_stride, const void* w, void* out,
+                   int64_t out_stride, int64_t rows, int hidden, float eps, hipStream_t stream) {
   if (rows == 0) return hipSuccess;
   hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)rows), dim3(kNormThreads), 0, stream,
-                     static_cast<const bf16*>(x), x_stride, static_cast<bf16*>(residual), r_stride,
+                     static_cast<const bf16*>(x), x_stride, static_cast<const bf16*>(residual),
+                     r_stride, static_cast<bf16*>(residual_out), ro_stride,
                      static_cast<const bf16*>(w), static_cast<bf16*>(out), out_stride, hidden, eps);
   return hipGetLastError();
 }

@@ -23,6 +23,62 @@ def _check_rows(t: torch.Tensor, name: str) -> None:
         raise ValueError(f"{name} must be a 2-D bfloat16 GPU tensor with contiguous rows")
 
 
+def _row_offsets_ok(h: torch.Tensor, residual: torch.Tensor | None, weight: torch.Tensor) -> bool:
+    """The operands lie within the 32-bit offsets of the folded RMSNorm's kernel."""
+    return (h.stride(0) <= 1 << 23 and (residual is None or residual.stride(0) <= 1 << 23)
+            and weight.shape[0] * weight.stride(0) < 1 << 30)
+
+
+def _plain_rows(t: torch.Tensor) -> bool:
+    """16-byte aligned, contiguous, non-overlapping rows."""
+    return (t.stride(1) == 1 and t.stride(0) >= t.shape[1] and t.stride(0) % 8 == 0
+            and t.data_ptr() % 16 == 0)
+
+
+def _add_rmsnorm(h: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
+                 eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """(RMSNorm(h + residual) * weight, h + residual), the inputs left unchanged."""
+    h = h if _plain_rows(h) else h.clone()
+    residual = residual if _plain_rows(residual) else residual.clone()
+    _check_rows(h, "x")
+    _check_rows(residual, "residual")
+    if h.shape != residual.shape:
+        raise ValueError("x and residual must have the same shape")
+    out, total = torch.empty_like(h), torch.empty_like(residual)
+    _lib.check(_lib.lib().aios_add_rmsnorm(
+        h.data_ptr(), h.stride(0), residual.data_ptr(), residual.stride(0), weight.data_ptr(),
+        total.data_ptr(), total.stride(0), out.data_ptr(), out.stride(0), h.shape[0], h.shape[1],
+        eps, _stream(h)), "aios_add_rmsnorm")
+    return out, total
+
+
+def _linear_rows(x: torch.Tensor, weight: torch.Tensor, n: int,
+                 residual: torch.Tensor | None = None, norm_weight: torch.Tensor | None = None,
+                 eps: float = 0.0, silu: bool = False):
+    """The few-row projection (aios_linear_rows_ws) to n columns, and with
+    norm_weight the residual-add RMSNorm folded in front of it: (y, h +
+    residual), the latter h itself without a residual."""
+    rows, k = x.shape
+    lib = _lib.lib()
+    y = torch.empty(rows, n, dtype=x.dtype, device=x.device)
+    norm = norm_weight is not None
+    total = torch.empty_like(x) if residual is not None else x
+    # (a buffer of this call alone: calls may overlap on several streams)
+    ws_bytes = 0 if norm or silu else lib.aios_linear_rows_workspace(rows, n, k)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+    _lib.check(lib.aios_linear_rows_ws(
+        x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), y.data_ptr(), y.stride(0),
+        rows, n, k, _lib.PROLOGUE_ADD_RMSNORM if norm else _lib.PROLOGUE_NONE,
+        residual.data_ptr() if residual is not None else None,
+        residual.stride(0) if residual is not None else 0,
+        norm_weight.data_ptr() if norm else None, eps,
+        total.data_ptr() if residual is not None else None,
+        total.stride(0) if residual is not None else 0,
+        _lib.EPILOGUE_SILU_MUL if silu else _lib.EPILOGUE_NONE,
+        ws.data_ptr() if ws is not None else None, ws_bytes, _stream(x)), "aios_linear_rows_ws")
+    return (y, total) if norm else y
+
+
 class HipOps:
     """RMSNorm, residual-add RMSNorm, q/k RMSNorm + RoPE, SiLU-and-mul, and
     the projections (few-row GEMM kernel for decode-sized inputs, the
@@ -43,11 +99,7 @@ class HipOps:
             return torch.nn.functional.linear(x, weight)
         if rows == 0:
             return x.new_empty(0, n)
-        y = torch.empty(rows, n, dtype=x.dtype, device=x.device)
-        _lib.check(_lib.lib().aios_linear_rows(x.data_ptr(), x.stride(0), weight.data_ptr(),
-                                               weight.stride(0), y.data_ptr(), y.stride(0), rows,
-                                               n, k, _stream(x)), "aios_linear_rows")
-        return y
+        return _linear_rows(x, weight, n)
 
     @staticmethod
     def _rows_ok(x: torch.Tensor, weight: torch.Tensor, k: int) -> bool:
@@ -66,33 +118,21 @@ class HipOps:
         (activation.py:9-12)."""
         rows, k = h.shape
         n = weight.shape[0] // 2 if silu else weight.shape[0]
-        # The prologue keeps (K/128) x (16-row tiles) normalised fragments in
-        # registers, at most 8: more rows than one launch holds run as row
-        # chunks (each re-reading the weights, mostly from L2) rather than
-        # as separate norm, projection and activation launches.
-        frags = (k // 4) // 32
-        chunk = 16 * (8 // frags) if 1 <= frags <= 8 else 0
-        if chunk and self._rows_ok(h, weight, k) and n % 16 == 0 and \
-                (residual is None or (residual.stride(1) == 1 and residual.stride(0) % 8 == 0)):
-            y = torch.empty(rows, n, dtype=h.dtype, device=h.device)
-            new_res = torch.empty_like(h) if residual is not None else h
-            lib = _lib.lib()
-            for r0 in range(0, rows, chunk):
-                m = min(chunk, rows - r0)
-                _lib.check(lib.aios_linear_rows_ex(
-                    h[r0:].data_ptr(), h.stride(0), weight.data_ptr(), weight.stride(0),
-                    y[r0:].data_ptr(), y.stride(0), m, n, k, _lib.PROLOGUE_ADD_RMSNORM,
-                    residual[r0:].data_ptr() if residual is not None else None,
-                    residual.stride(0) if residual is not None else 0, norm_weight.data_ptr(),
-                    eps, new_res[r0:].data_ptr() if residual is not None else None,
-                    new_res.stride(0) if residual is not None else 0,
-                    _lib.EPILOGUE_SILU_MUL if silu else _lib.EPILOGUE_NONE, _stream(h)),
-                    "aios_linear_rows_ex")
-            return y, new_res
+        rows_ok = self._rows_ok(h, weight, k) and n % 16 == 0
+        # (up to K = 1024 the kernel's own checks judge the operands; wider rows
+        # it does not take as they are go through the separate norm)
+        if (rows_ok and rows <= 32 and k <= 2560 and _row_offsets_ok(h, residual, weight)
+                and (residual is None
+                     or (residual.stride(1) == 1 and residual.stride(0) % 8 == 0))
+                and (k <= 1024 or (_plain_rows(h)
+                                   and (residual is None or _plain_rows(residual))))):
+            return _linear_rows(h, weight, n, residual, norm_weight, eps, silu)
         if residual is None:
             x, residual = self.rmsnorm(h, norm_weight, eps), h
-        else:  # (the inputs are left unchanged, as on the folded path)
-            x, residual = self.fused_add_rmsnorm(h.clone(), residual.clone(), norm_weight, eps)
+        else:
+            x, residual = _add_rmsnorm(h, residual, norm_weight, eps)
+        if silu and rows_ok and k <= 2560:
+            return _linear_rows(x, weight, n, silu=True), residual
         y = self.linear(x, weight)
         return (self.silu_and_mul(y) if silu else y), residual
 

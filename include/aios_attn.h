@@ -304,6 +304,16 @@ int aios_rmsnorm(const void* x, int64_t x_stride, void* residual, int64_t residu
                  float eps, void* stream);
 
 /*
+ * The residual form of aios_rmsnorm with its own output for the sum:
+ * residual_out = bf16(x + residual), out = bf16(RMSNorm(x + residual) *
+ * weight); x and residual are left as they are (residual_out may alias
+ * residual, out may alias x).
+ */
+int aios_add_rmsnorm(const void* x, int64_t x_stride, const void* residual, int64_t residual_stride,
+                     const void* weight, void* residual_out, int64_t residual_out_stride, void* out,
+                     int64_t out_stride, int64_t rows, int32_t hidden, float eps, void* stream);
+
+/*
  * Per-head query/key RMSNorm followed by rotary embedding, from the fused
  * qkv projection rows [tokens][(Hq + 2*Hkv) * D] (row stride qkv_stride):
  *   x' = bf16(x * rsqrt(mean(x^2) + eps) * w)                (q or k weight)
@@ -366,6 +376,22 @@ int aios_linear_rows_ex(const void* x, int64_t x_stride, const void* weight, int
                         int64_t residual_stride, const void* norm_weight, float eps,
                         void* residual_out, int64_t residual_out_stride, int32_t epilogue,
                         void* stream);
+
+/*
+ * aios_linear_rows_ex with a workspace (16-byte aligned), in which a long
+ * in_features is split over groups of workgroups when it holds the
+ * aios_linear_rows_workspace(...) bytes of fp32 partial products (0: none
+ * used; a smaller or null workspace runs unsplit).  The RMSNorm prologue is
+ * supported for up to 32 rows with in_features up to 2560, besides the
+ * shapes of aios_linear_rows_ex.
+ */
+int64_t aios_linear_rows_workspace(int64_t rows, int64_t out_features, int64_t in_features);
+int aios_linear_rows_ws(const void* x, int64_t x_stride, const void* weight, int64_t w_stride,
+                        void* y, int64_t y_stride, int64_t rows, int64_t out_features,
+                        int64_t in_features, int32_t prologue, const void* residual,
+                        int64_t residual_stride, const void* norm_weight, float eps,
+                        void* residual_out, int64_t residual_out_stride, int32_t epilogue,
+                        void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * The per-step bookkeeping of a captured CandidateGroup decode step (the

@@ -151,3 +151,60 @@ def test_add_rmsnorm_linear_silu_pair(rows, k, inter, with_residual):
     y_ref = ref.silu_and_mul(gu).float()
     err = (y.float() - y_ref).abs()
     assert bool((err <= 2.0 ** -6 * y_ref.abs() + 4e-3 * y_ref.abs().max()).all()), err.max().item()
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 16, 256), (24, 2560, 4096), (32, 48, 3072), (33, 2560, 9728),
+                                   (48, 1024, 2560), (49, 272, 1280), (64, 20016, 2560),
+                                   (64, 768, 2048), (1, 2560, 9728), (9, 6144, 2560),
+                                   (16, 32, 4224), (24, 40000, 768)])
+def test_streaming_rows_match_fp32_gemm(m, n, k):
+    """The resident-row streaming GEMM: each count of 16-row tiles, one tile
+    and many per workgroup, K split over workgroups (with a remainder of K
+    steps), columns that do not divide over the workgroups.  fp32 sums, one
+    bf16 rounding (2^-9 of the value) plus the sums' own error, bounded by
+    k * 2^-24 of the magnitudes summed."""
+    x = _bf16((m, k), m + k, 1.0)
+    w = _bf16((n, k), n, 0.05)
+    y = HipOps().linear(x, w).double()
+    ref = x.double() @ w.double().T
+    bound = 2.0 ** -8 * ref.abs() + k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((y - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("rows,k,n", [(17, 768, 6144), (32, 2560, 512), (9, 2560, 4864),
+                                      (24, 1280, 48), (24, 2304, 16), (40, 2560, 256),
+                                      (64, 1024, 3072)])
+@pytest.mark.parametrize("silu", [True, False])
+@pytest.mark.parametrize("with_residual", [True, False])
+def test_streaming_rows_norm_and_silu(rows, k, n, silu, with_residual):
+    h = _bf16((rows, k), rows + k, 2.0)
+    r = _bf16((rows, k), rows + k + 1, 3.0) if with_residual else None
+    nw = _bf16((k,), 9).abs() + 0.5
+    w = _bf16((2 * n if silu else n, k), n, 0.05)
+    y, new_r = HipOps().add_rmsnorm_linear(h, r, nw, 1e-6, w, silu=silu)
+    ref = TorchOps()
+    if with_residual:
+        x_ref, r_ref = ref.fused_add_rmsnorm(h.clone(), r.clone(), nw, 1e-6)
+        assert torch.equal(new_r, r_ref)
+    else:
+        x_ref = ref.rmsnorm(h, nw, 1e-6)
+        assert new_r is h
+    y_ref = x_ref.float() @ w.float().T
+    if silu:
+        y_ref = ref.silu_and_mul(y_ref.to(torch.bfloat16)).float()
+    err = (y.float() - y_ref).abs()
+    tol = 2.0 ** -6 if silu else 2.0 ** -7
+    assert bool((err <= tol * y_ref.abs() + 4e-3 * y_ref.abs().max()).all()), err.max().item()
+
+
+def test_norm_takes_rows_it_cannot_read_in_place():
+    """Wide rows with an odd offset, an odd stride or a column stride are copied
+    for the separate norm, as before the norm read its inputs in place."""
+    big = _bf16((8, 2 * 2560 + 24), 11, 1.0)
+    r = _bf16((8, 2560), 12, 1.0)
+    nw, w = _bf16((2560,), 13).abs() + 0.5, _bf16((64, 2560), 14, 0.05)
+    for h in (big[:, 4:2564], big[:, ::2][:, :2560], big[:1, :2560].expand(8, 2560)):
+        y, total = HipOps().add_rmsnorm_linear(h, r, nw, 1e-6, w)
+        y_ref, t_ref = HipOps().add_rmsnorm_linear(h.contiguous(), r, nw, 1e-6, w)
+        assert torch.equal(total, t_ref)
+        torch.testing.assert_close(y.float(), y_ref.float(), atol=2e-2, rtol=2e-2)
