@@ -173,7 +173,7 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.aios_linear_rows_workspace.argtypes = [_i64, _i64, _i64]
     lib.aios_linear_rows_ws.restype = ctypes.c_int
     lib.aios_linear_rows_ws.argtypes = [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i32,
-                                        _vp, _i64, _vp, _f32, _vp, _i64, _i32, _vp, _i64, _vp]
+                                        _vp, _i64, _vp]
     lib.aios_linear_rows_ex.restype = ctypes.c_int
     lib.aios_linear_rows_ex.argtypes = [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i32,
                                         _vp, _i64, _vp, _f32, _vp, _i64, _i32, _vp]

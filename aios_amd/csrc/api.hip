@@ -75,8 +75,8 @@ int device_cus() {
 // 16-row tile, or a K without a fixed-K instance in gemm_skinny.hip, which
 // are the faster ones where they exist (8 rows, N x K 4096 x 1024: 3.9 us
 // against 5.0; 1024 x 2048: 4.4 against 6.0).
-bool rows_form(int64_t rows, int64_t k, bool norm) {
-  return rows > 16 || (k > 1024 && (norm || (k != 2048 && k != 3072)));
+bool rows_form(int64_t rows, int64_t k) {
+  return rows > 16 || (k > 1024 && k != 2048 && k != 3072);
 }
 
 // How a prefill batch splits its tiles' KV ranges over workgroups
@@ -719,31 +719,6 @@ int aios_linear_rows_ex(const void* x, int64_t x_stride, const void* weight, int
                         int64_t residual_stride, const void* norm_weight, float eps,
                         void* residual_out, int64_t residual_out_stride, int32_t epilogue,
                         void* stream) {
-  if (prologue == AIOS_PROLOGUE_ADD_RMSNORM &&
-      aios::skinny_gemm_supported(rows, out_features, in_features) &&
-      !aios::skinny_gemm_norm_supported(rows, in_features))
-    return fail(AIOS_ERR_UNSUPPORTED, "linear_rows: RMSNorm prologue for %lld rows x %lld",
-                (long long)rows, (long long)in_features);
-  return aios_linear_rows_ws(x, x_stride, weight, w_stride, y, y_stride, rows, out_features,
-                             in_features, prologue, residual, residual_stride, norm_weight, eps,
-                             residual_out, residual_out_stride, epilogue, nullptr, 0, stream);
-}
-
-int64_t aios_linear_rows_workspace(int64_t rows, int64_t out_features, int64_t in_features) {
-  aios::RowsPlan p;
-  if (!aios::skinny_gemm_supported(rows, out_features, in_features) ||
-      !rows_form(rows, in_features, false) ||
-      !aios::rows_gemm_plan(rows, out_features, in_features, false, false, true, device_cus(), &p))
-    return 0;
-  return p.bytes;
-}
-
-int aios_linear_rows_ws(const void* x, int64_t x_stride, const void* weight, int64_t w_stride,
-                        void* y, int64_t y_stride, int64_t rows, int64_t out_features,
-                        int64_t in_features, int32_t prologue, const void* residual,
-                        int64_t residual_stride, const void* norm_weight, float eps,
-                        void* residual_out, int64_t residual_out_stride, int32_t epilogue,
-                        void* workspace, int64_t workspace_bytes, void* stream) {
   if (!aios::skinny_gemm_supported(rows, out_features, in_features))
     return fail(AIOS_ERR_UNSUPPORTED,
                 "linear_rows: needs 1..64 rows, out_features %% 16 == 0, in_features %% 128 == 0 "
@@ -753,6 +728,9 @@ int aios_linear_rows_ws(const void* x, int64_t x_stride, const void* weight, int
     return fail(AIOS_ERR_INVALID, "linear_rows: unknown prologue %d", prologue);
   if (epilogue != AIOS_EPILOGUE_NONE && epilogue != AIOS_EPILOGUE_SILU_MUL)
     return fail(AIOS_ERR_INVALID, "linear_rows: unknown epilogue %d", epilogue);
+  if (prologue == AIOS_PROLOGUE_ADD_RMSNORM && !aios::skinny_gemm_norm_supported(rows, in_features))
+    return fail(AIOS_ERR_UNSUPPORTED, "linear_rows: RMSNorm prologue for %lld rows x %lld",
+                (long long)rows, (long long)in_features);
   if (!x || !weight || !y) return fail(AIOS_ERR_INVALID, "linear_rows: null pointer");
   if (x_stride < in_features || w_stride < in_features || y_stride < out_features ||
       (x_stride | w_stride) % 8 != 0 || y_stride % 4 != 0)
@@ -771,6 +749,9 @@ int aios_linear_rows_ws(const void* x, int64_t x_stride, const void* weight, int
     if (residual_out && (residual_out == x || residual_out == residual))
       return fail(AIOS_ERR_INVALID, "linear_rows: residual_out must not alias the inputs");
   }
+  if (prologue == AIOS_PROLOGUE_NONE)
+    return aios_linear_rows_ws(x, x_stride, weight, w_stride, y, y_stride, rows, out_features,
+                               in_features, epilogue, nullptr, 0, stream);
   aios::LinearArgs a = {};
   a.x = static_cast<const aios::bf16*>(x);
   a.x_stride = x_stride;
@@ -787,24 +768,57 @@ int aios_linear_rows_ws(const void* x, int64_t x_stride, const void* weight, int
   a.eps = eps;
   a.residual_out = static_cast<aios::bf16*>(residual_out);
   a.ro_stride = residual_out_stride;
-  const bool norm = prologue == AIOS_PROLOGUE_ADD_RMSNORM;
-  const bool silu = epilogue == AIOS_EPILOGUE_SILU_MUL;
-  if (rows_form(rows, in_features, norm) && aios::rows_gemm_fits(a, silu)) {
-    const bool ws = workspace && ((uintptr_t)workspace & 15) == 0;
-    aios::RowsPlan p;
-    bool ok = aios::rows_gemm_plan(rows, out_features, in_features, norm, silu, ws, device_cus(), &p);
-    if (ok && p.bytes > workspace_bytes)
-      ok = aios::rows_gemm_plan(rows, out_features, in_features, norm, silu, false, device_cus(), &p);
-    if (ok)
-      return check_hip(aios::rows_gemm(a, norm, silu, p, workspace,
-                                       static_cast<hipStream_t>(stream)),
-                       "linear_rows launch");
-  }
-  if (norm && !aios::skinny_gemm_norm_supported(rows, in_features))
-    return fail(AIOS_ERR_UNSUPPORTED, "linear_rows: RMSNorm prologue for %lld rows x %lld",
-                (long long)rows, (long long)in_features);
   return check_hip(aios::skinny_gemm(a, prologue, epilogue, static_cast<hipStream_t>(stream)),
                    "linear_rows launch");
+}
+
+int64_t aios_linear_rows_workspace(int64_t rows, int64_t out_features, int64_t in_features) {
+  aios::RowsPlan p;
+  if (!aios::skinny_gemm_supported(rows, out_features, in_features) ||
+      !rows_form(rows, in_features) ||
+      !aios::rows_gemm_plan(rows, out_features, in_features, false, true, device_cus(), &p))
+    return 0;
+  return p.bytes;
+}
+
+int aios_linear_rows_ws(const void* x, int64_t x_stride, const void* weight, int64_t w_stride,
+                        void* y, int64_t y_stride, int64_t rows, int64_t out_features,
+                        int64_t in_features, int32_t epilogue, void* workspace,
+                        int64_t workspace_bytes, void* stream) {
+  if (!aios::skinny_gemm_supported(rows, out_features, in_features))
+    return fail(AIOS_ERR_UNSUPPORTED,
+                "linear_rows: needs 1..64 rows, out_features %% 16 == 0, in_features %% 128 == 0 "
+                "(got %lld x %lld x %lld)",
+                (long long)rows, (long long)out_features, (long long)in_features);
+  if (epilogue != AIOS_EPILOGUE_NONE && epilogue != AIOS_EPILOGUE_SILU_MUL)
+    return fail(AIOS_ERR_INVALID, "linear_rows: unknown epilogue %d", epilogue);
+  if (!x || !weight || !y) return fail(AIOS_ERR_INVALID, "linear_rows: null pointer");
+  if (x_stride < in_features || w_stride < in_features || y_stride < out_features ||
+      (x_stride | w_stride) % 8 != 0 || y_stride % 4 != 0)
+    return fail(AIOS_ERR_INVALID, "linear_rows: bad row strides");
+  if ((((uintptr_t)x | (uintptr_t)weight) & 15) != 0 || ((uintptr_t)y & 7) != 0)
+    return fail(AIOS_ERR_INVALID, "linear_rows: misaligned rows");
+  aios::LinearArgs a = {};
+  a.x = static_cast<const aios::bf16*>(x);
+  a.x_stride = x_stride;
+  a.w = static_cast<const aios::bf16*>(weight);
+  a.w_stride = w_stride;
+  a.y = static_cast<aios::bf16*>(y);
+  a.y_stride = y_stride;
+  a.M = (int32_t)rows;
+  a.K = (int32_t)in_features;
+  a.N = out_features;
+  const bool silu = epilogue == AIOS_EPILOGUE_SILU_MUL;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (rows_form(rows, in_features) && aios::rows_gemm_fits(a, silu)) {
+    const bool ws = workspace && ((uintptr_t)workspace & 15) == 0;
+    aios::RowsPlan p;
+    bool ok = aios::rows_gemm_plan(rows, out_features, in_features, silu, ws, device_cus(), &p);
+    if (ok && p.bytes > workspace_bytes)
+      ok = aios::rows_gemm_plan(rows, out_features, in_features, silu, false, device_cus(), &p);
+    if (ok) return check_hip(aios::rows_gemm(a, silu, p, workspace, s), "linear_rows launch");
+  }
+  return check_hip(aios::skinny_gemm(a, AIOS_PROLOGUE_NONE, epilogue, s), "linear_rows launch");
 }
 
 int aios_cg_step_begin(int64_t* step, const int32_t* pages, int32_t page_rows, int32_t rows,

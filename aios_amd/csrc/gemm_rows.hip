@@ -20,10 +20,11 @@
 // 40 -> 24, 2560 x 4096 19.2 -> 9.7 (4 splits), 2560 x 9728 42 -> 15.7 (8
 // splits); 64 rows, 2560 x 9728 60 -> 20; 8 rows, 151936 x 2560 192 -> 141.
 //
-// Prologue kAddNorm (splits = 1): x = bf16(RMSNorm(x + residual) * norm_w) as
-// in gemm_skinny.hip, formed once per workgroup in the registers, workgroup
-// 0 writing bf16(x + residual).  Epilogue kSiluPair: a tile is 8 gate columns
-// and the 8 matching up columns, so the pair meets in one wavefront.
+// With SILU (gate rows, then up rows in W: the merged gate/up projection) a
+// tile is 8 gate columns and the 8 matching up columns, so the pair meets in
+// one wavefront.  The residual-add RMSNorm is not folded in here: every
+// workgroup would normalise all rows (24 rows x 6144 x 2560: 24 us against 15
+// with the norm as its own launch; 24 x 4096 x 1024: 8.5 against 8.0).
 #include "kernels.hpp"
 
 namespace aios {
@@ -40,14 +41,6 @@ constexpr int64_t kRange = 0x7fffffff;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-struct RowsNorm {
-  const bf16* residual;  // may be null
-  const bf16* norm_w;
-  bf16* residual_out;  // may be null
-  int32_t r_stride, ro_stride;
-  float eps;
-};
-
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_buffer(const void* p) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)kRange, kRsrcWord3);
 }
@@ -59,17 +52,16 @@ __device__ __forceinline__ bf16x8 rows_load(__amdgpu_buffer_rsrc_t r, int voff, 
 // serve where MT * KS fragments leave no room for two of KS.
 // Register use at two wavefronts per SIMD (256): 4 * (MT * KS + 2 * KS / NH)
 // for the fragments, at most 240.
-template <int MT, int KS, int NH, bool NORM, bool SILU, bool PART>
+template <int MT, int KS, int NH, bool SILU, bool PART>
 __global__ __launch_bounds__(kRowsThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void rows_gemm_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* __restrict__ y, int32_t x_stride,
     int32_t w_stride, int32_t y_stride, int32_t M, int32_t K, int32_t N, int32_t splits,
-    float* __restrict__ part, RowsNorm nrm) {
-  static_assert(!PART || (!NORM && !SILU), "partial tiles are sums only");
+    float* __restrict__ part) {
+  static_assert(!PART || !SILU, "partial tiles are sums only");
   static_assert(NH <= 2 && KS % NH == 0, "one or two halves");
   constexpr int KH = KS / NH;
   constexpr int NC = SILU ? 8 : 16;  // output columns of a tile
   __shared__ f32x4 red[2][kRowsWaves][MT][64];
-  __shared__ float ssq[kRowsWaves][MT][16];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15;
@@ -109,64 +101,6 @@ __global__ __launch_bounds__(kRowsThreads) __attribute__((amdgpu_waves_per_eu(2,
         xb[mt][u] = rows_load(rx, u < ns ? off : kOut, (s0 + min(u, ns - 1)) * 64);
     }
   }
-  if constexpr (NORM) {
-    const __amdgpu_buffer_rsrc_t rr = rows_buffer(nrm.residual);
-    bf16x8 rb[MT][KS];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = mt * 16 + l16;
-      const int off = m < M && nrm.residual ? (m * nrm.r_stride + lg * 8) * 2 : kOut;
-#pragma unroll
-      for (int u = 0; u < KS; ++u)
-        rb[mt][u] = rows_load(rr, u < ns ? off : kOut, (s0 + min(u, ns - 1)) * 64);
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      float ss = 0.f;
-#pragma unroll
-      for (int u = 0; u < KS; ++u) {
-        float a[8], b[8];
-        unpack_bf16x8(xb[mt][u], a);
-        unpack_bf16x8(rb[mt][u], b);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          a[j] += b[j];
-          ss = fmaf(a[j], a[j], ss);
-        }
-        const int m = mt * 16 + l16;
-        if (nrm.residual_out && blockIdx.x == 0 && m < M && u < ns)
-          *reinterpret_cast<bf16x8*>(nrm.residual_out + (int64_t)m * nrm.ro_stride + (s0 + u) * 32 +
-                                     lg * 8) = pack_bf16x8(a);
-      }
-      ss = xrow_sum(ss);
-      if (lg == 0) ssq[wave][mt][l16] = ss;
-    }
-    __syncthreads();
-    float inv[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      float ss = 0.f;
-#pragma unroll
-      for (int q = 0; q < kRowsWaves; ++q) ss += ssq[q][mt][l16];
-      inv[mt] = rsqrtf(ss / (float)K + nrm.eps);
-    }
-    const __amdgpu_buffer_rsrc_t rn = rows_buffer(nrm.norm_w);
-#pragma unroll
-    for (int u = 0; u < KS; ++u) {
-      float nw[8];
-      unpack_bf16x8(rows_load(rn, lg * 16, (s0 + min(u, ns - 1)) * 64), nw);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        float a[8], b[8];
-        unpack_bf16x8(xb[mt][u], a);
-        unpack_bf16x8(rb[mt][u], b);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) a[j] = (a[j] + b[j]) * inv[mt] * nw[j];
-        xb[mt][u] = pack_bf16x8(a);
-      }
-    }
-  }
-
   f32x4 acc[MT];
   auto mma = [&](const bf16x8 (&f)[KH], int half) {
 #pragma unroll
@@ -282,65 +216,53 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(const float* __restric
 
 // The register steps built for a row tile count, 0 when the K steps per
 // wavefront do not fit.
-int rows_ks(int mt, int need, bool norm, bool silu) {
+int rows_ks(int mt, int need, bool silu) {
   if (need <= 3) return 3;
   if (need <= 4) return 4;
   if (need <= 6) return silu ? 8 : 6;
   if (need <= 8) return 8;
   if (need <= 10) return 10;
-  if (need <= 12 && mt <= 2 && !norm && !silu) return 12;
+  if (need <= 12 && mt <= 2 && !silu) return 12;
   return 0;
 }
 
 template <int MT, int KS, int NH = 1>
-hipError_t launch_rows(const LinearArgs& a, bool norm, bool silu, const RowsPlan& p, float* part,
+hipError_t launch_rows(const LinearArgs& a, bool silu, const RowsPlan& p, float* part,
                        hipStream_t stream) {
-  const RowsNorm n = {a.residual, a.norm_w, a.residual_out, (int32_t)a.r_stride,
-                      (int32_t)a.ro_stride, a.eps};
-#define AIOS_ROWS(NORM, SILU, PART)                                                              \
-  hipLaunchKernelGGL((rows_gemm_kernel<MT, KS, NH, NORM, SILU, PART>), dim3((unsigned)p.grid),   \
+#define AIOS_ROWS(SILU, PART)                                                                    \
+  hipLaunchKernelGGL((rows_gemm_kernel<MT, KS, NH, SILU, PART>), dim3((unsigned)p.grid),         \
                      dim3(kRowsThreads), 0, stream, a.x, a.w, a.y, (int32_t)a.x_stride,          \
                      (int32_t)a.w_stride, (int32_t)a.y_stride, a.M, a.K, (int32_t)a.N, p.splits, \
-                     part, n)
+                     part)
   if (p.splits > 1) {
-    AIOS_ROWS(false, false, true);
+    AIOS_ROWS(false, true);
     const int64_t quads = (int64_t)a.M * (a.N / 4);
     hipLaunchKernelGGL(rows_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0,
                        stream, part, a.y, p.splits, a.M, (int32_t)a.N, (int32_t)a.y_stride);
     return hipGetLastError();
   }
-  if constexpr (MT <= 2 && KS <= 10) {
-    if (norm) {
-      if (silu) {
-        if constexpr (KS != 6) AIOS_ROWS(true, true, false);
-      } else {
-        AIOS_ROWS(true, false, false);
-      }
-      return hipGetLastError();
-    }
-  }
   if constexpr (KS != 6 && KS != 12) {
     if (silu) {
-      AIOS_ROWS(false, true, false);
+      AIOS_ROWS(true, false);
       return hipGetLastError();
     }
   }
-  AIOS_ROWS(false, false, false);
+  AIOS_ROWS(false, false);
 #undef AIOS_ROWS
   return hipGetLastError();
 }
 
 template <int MT>
-hipError_t launch_rows_mt(const LinearArgs& a, bool norm, bool silu, const RowsPlan& p, float* part,
+hipError_t launch_rows_mt(const LinearArgs& a, bool silu, const RowsPlan& p, float* part,
                           hipStream_t stream) {
   switch (p.ks) {
-    case 3: return launch_rows<MT, 3>(a, norm, silu, p, part, stream);
-    case 4: return launch_rows<MT, 4>(a, norm, silu, p, part, stream);
-    case 6: return launch_rows<MT, 6>(a, norm, silu, p, part, stream);
-    case 8: return launch_rows<MT, 8>(a, norm, silu, p, part, stream);
-    case 10: return launch_rows<MT, 10, MT == 4 ? 2 : 1>(a, norm, silu, p, part, stream);
+    case 3: return launch_rows<MT, 3>(a, silu, p, part, stream);
+    case 4: return launch_rows<MT, 4>(a, silu, p, part, stream);
+    case 6: return launch_rows<MT, 6>(a, silu, p, part, stream);
+    case 8: return launch_rows<MT, 8>(a, silu, p, part, stream);
+    case 10: return launch_rows<MT, 10, MT == 4 ? 2 : 1>(a, silu, p, part, stream);
     case 12:
-      if constexpr (MT <= 2) return launch_rows<MT, 12>(a, norm, silu, p, part, stream);
+      if constexpr (MT <= 2) return launch_rows<MT, 12>(a, silu, p, part, stream);
       break;
     default: break;
   }
@@ -357,18 +279,17 @@ hipError_t launch_rows_mt(const LinearArgs& a, bool norm, bool silu, const RowsP
 // takes 1 split for 6144 x 2560 (12 us, 2 splits 12.7), 6 for 2560 x 4096
 // (9.6; 2 splits 10.9), 8 for 2560 x 9728 (15.7; 4 splits 17.7) and 4 for
 // 1024 x 3072 (6.7 us; unsplit 9 in the eight-column skinny form).
-bool rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool norm, bool silu, bool workspace, int cus,
+bool rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool silu, bool workspace, int cus,
                     RowsPlan* plan) {
   if (M < 1 || M > 64 || N < 16 || N % 16 != 0 || K < 256 || K % 32 != 0 || K > (1 << 20))
     return false;
   const int mt = (int)((M + 15) / 16);
-  if (norm && mt > 2) return false;
   const int64_t T = K / 32, nc = silu ? 8 : 16, tiles = N / nc;
   double best = 0.0;
   plan->splits = 0;
-  for (int s = 1; s <= (workspace && !norm && !silu ? kRowsMaxSplits : 1); ++s) {
+  for (int s = 1; s <= (workspace && !silu ? kRowsMaxSplits : 1); ++s) {
     if (T < kRowsWaves * s) break;
-    const int ks = rows_ks(mt, (int)((T + kRowsWaves * s - 1) / (kRowsWaves * s)), norm, silu);
+    const int ks = rows_ks(mt, (int)((T + kRowsWaves * s - 1) / (kRowsWaves * s)), silu);
     if (ks == 0) continue;
     const int64_t C = tiles < cus / s ? tiles : cus / s;
     const int64_t walk = (tiles + C - 1) / C;
@@ -386,14 +307,13 @@ bool rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool norm, bool silu, bool 
   return plan->bytes < kRange;
 }
 
-hipError_t rows_gemm(const LinearArgs& a, bool norm, bool silu, const RowsPlan& p, void* workspace,
-                     hipStream_t stream) {
+hipError_t rows_gemm(const LinearArgs& a, bool silu, const RowsPlan& p, void* workspace, hipStream_t stream) {
   float* part = static_cast<float*>(workspace);
   switch ((a.M + 15) / 16) {
-    case 1: return launch_rows_mt<1>(a, norm, silu, p, part, stream);
-    case 2: return launch_rows_mt<2>(a, norm, silu, p, part, stream);
-    case 3: return launch_rows_mt<3>(a, norm, silu, p, part, stream);
-    case 4: return launch_rows_mt<4>(a, norm, silu, p, part, stream);
+    case 1: return launch_rows_mt<1>(a, silu, p, part, stream);
+    case 2: return launch_rows_mt<2>(a, silu, p, part, stream);
+    case 3: return launch_rows_mt<3>(a, silu, p, part, stream);
+    case 4: return launch_rows_mt<4>(a, silu, p, part, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -401,8 +321,8 @@ hipError_t rows_gemm(const LinearArgs& a, bool norm, bool silu, const RowsPlan& 
 // Offsets inside each operand are 32-bit.
 bool rows_gemm_fits(const LinearArgs& a, bool silu) {
   const int64_t w_rows = (silu ? 2 : 1) * a.N;
-  return a.x_stride <= (1 << 23) && a.y_stride <= (1 << 23) && a.r_stride <= (1 << 23) &&
-         a.ro_stride <= (1 << 23) && w_rows * a.w_stride * 2 < kRange && a.N <= (1 << 23);
+  return a.x_stride <= (1 << 23) && a.y_stride <= (1 << 23) &&
+         w_rows * a.w_stride * 2 < kRange && a.N <= (1 << 23);
 }
 
 }  // namespace aios

@@ -222,10 +222,10 @@ struct RowsPlan {
   int32_t splits, ks, grid;
   int64_t bytes;
 };
-bool rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool norm, bool silu, bool workspace, int cus,
+bool rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool silu, bool workspace, int cus,
                     RowsPlan* plan);
 bool rows_gemm_fits(const LinearArgs& a, bool silu);
-hipError_t rows_gemm(const LinearArgs& a, bool norm, bool silu, const RowsPlan& p, void* workspace,
+hipError_t rows_gemm(const LinearArgs& a, bool silu, const RowsPlan& p, void* workspace,
                      hipStream_t stream);
 
 hipError_t greedy_select(const void* logits, int64_t row_stride, int32_t rows, int32_t vocab,

@@ -23,12 +23,6 @@ def _check_rows(t: torch.Tensor, name: str) -> None:
         raise ValueError(f"{name} must be a 2-D bfloat16 GPU tensor with contiguous rows")
 
 
-def _row_offsets_ok(h: torch.Tensor, residual: torch.Tensor | None, weight: torch.Tensor) -> bool:
-    """The operands lie within the 32-bit offsets of the folded RMSNorm's kernel."""
-    return (h.stride(0) <= 1 << 23 and (residual is None or residual.stride(0) <= 1 << 23)
-            and weight.shape[0] * weight.stride(0) < 1 << 30)
-
-
 def _plain_rows(t: torch.Tensor) -> bool:
     """16-byte aligned, contiguous, non-overlapping rows."""
     return (t.stride(1) == 1 and t.stride(0) >= t.shape[1] and t.stride(0) % 8 == 0
@@ -52,31 +46,19 @@ def _add_rmsnorm(h: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
     return out, total
 
 
-def _linear_rows(x: torch.Tensor, weight: torch.Tensor, n: int,
-                 residual: torch.Tensor | None = None, norm_weight: torch.Tensor | None = None,
-                 eps: float = 0.0, silu: bool = False):
-    """The few-row projection (aios_linear_rows_ws) to n columns, and with
-    norm_weight the residual-add RMSNorm folded in front of it: (y, h +
-    residual), the latter h itself without a residual."""
+def _linear_rows(x: torch.Tensor, weight: torch.Tensor, n: int, silu: bool = False) -> torch.Tensor:
+    """The few-row projection (aios_linear_rows_ws) to n columns."""
     rows, k = x.shape
     lib = _lib.lib()
     y = torch.empty(rows, n, dtype=x.dtype, device=x.device)
-    norm = norm_weight is not None
-    total = torch.empty_like(x) if residual is not None else x
     # (a buffer of this call alone: calls may overlap on several streams)
-    ws_bytes = 0 if norm or silu else lib.aios_linear_rows_workspace(rows, n, k)
+    ws_bytes = 0 if silu else lib.aios_linear_rows_workspace(rows, n, k)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     _lib.check(lib.aios_linear_rows_ws(
         x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), y.data_ptr(), y.stride(0),
-        rows, n, k, _lib.PROLOGUE_ADD_RMSNORM if norm else _lib.PROLOGUE_NONE,
-        residual.data_ptr() if residual is not None else None,
-        residual.stride(0) if residual is not None else 0,
-        norm_weight.data_ptr() if norm else None, eps,
-        total.data_ptr() if residual is not None else None,
-        total.stride(0) if residual is not None else 0,
-        _lib.EPILOGUE_SILU_MUL if silu else _lib.EPILOGUE_NONE,
+        rows, n, k, _lib.EPILOGUE_SILU_MUL if silu else _lib.EPILOGUE_NONE,
         ws.data_ptr() if ws is not None else None, ws_bytes, _stream(x)), "aios_linear_rows_ws")
-    return (y, total) if norm else y
+    return y
 
 
 class HipOps:
@@ -119,14 +101,25 @@ class HipOps:
         rows, k = h.shape
         n = weight.shape[0] // 2 if silu else weight.shape[0]
         rows_ok = self._rows_ok(h, weight, k) and n % 16 == 0
-        # (up to K = 1024 the kernel's own checks judge the operands; wider rows
-        # it does not take as they are go through the separate norm)
-        if (rows_ok and rows <= 32 and k <= 2560 and _row_offsets_ok(h, residual, weight)
+        # One 16-row tile whose normalised fragments fit the registers (K / 128
+        # of them, at most 8) takes the norm in the projection's launch; more
+        # rows pay less for it as a launch of its own than for forming it in
+        # every workgroup (24 x 768 x 1280: 6.7 us against 9 in two tiles).
+        if (rows_ok and rows <= 16 and k <= 1024
                 and (residual is None
-                     or (residual.stride(1) == 1 and residual.stride(0) % 8 == 0))
-                and (k <= 1024 or (_plain_rows(h)
-                                   and (residual is None or _plain_rows(residual))))):
-            return _linear_rows(h, weight, n, residual, norm_weight, eps, silu)
+                     or (residual.stride(1) == 1 and residual.stride(0) % 8 == 0))):
+            y = torch.empty(rows, n, dtype=h.dtype, device=h.device)
+            total = torch.empty_like(h) if residual is not None else h
+            _lib.check(_lib.lib().aios_linear_rows_ex(
+                h.data_ptr(), h.stride(0), weight.data_ptr(), weight.stride(0), y.data_ptr(),
+                y.stride(0), rows, n, k, _lib.PROLOGUE_ADD_RMSNORM,
+                residual.data_ptr() if residual is not None else None,
+                residual.stride(0) if residual is not None else 0, norm_weight.data_ptr(), eps,
+                total.data_ptr() if residual is not None else None,
+                total.stride(0) if residual is not None else 0,
+                _lib.EPILOGUE_SILU_MUL if silu else _lib.EPILOGUE_NONE, _stream(h)),
+                "aios_linear_rows_ex")
+            return y, total
         if residual is None:
             x, residual = self.rmsnorm(h, norm_weight, eps), h
         else:

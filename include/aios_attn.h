@@ -378,20 +378,16 @@ int aios_linear_rows_ex(const void* x, int64_t x_stride, const void* weight, int
                         void* stream);
 
 /*
- * aios_linear_rows_ex with a workspace (16-byte aligned), in which a long
- * in_features is split over groups of workgroups when it holds the
- * aios_linear_rows_workspace(...) bytes of fp32 partial products (0: none
- * used; a smaller or null workspace runs unsplit).  The RMSNorm prologue is
- * supported for up to 32 rows with in_features up to 2560, besides the
- * shapes of aios_linear_rows_ex.
+ * aios_linear_rows (epilogue as in aios_linear_rows_ex) with a workspace,
+ * 16-byte aligned: a long in_features is split over groups of workgroups
+ * when it holds the aios_linear_rows_workspace(...) bytes of fp32 partial
+ * products (0: none used; a smaller or null workspace runs unsplit).
  */
 int64_t aios_linear_rows_workspace(int64_t rows, int64_t out_features, int64_t in_features);
 int aios_linear_rows_ws(const void* x, int64_t x_stride, const void* weight, int64_t w_stride,
                         void* y, int64_t y_stride, int64_t rows, int64_t out_features,
-                        int64_t in_features, int32_t prologue, const void* residual,
-                        int64_t residual_stride, const void* norm_weight, float eps,
-                        void* residual_out, int64_t residual_out_stride, int32_t epilogue,
-                        void* workspace, int64_t workspace_bytes, void* stream);
+                        int64_t in_features, int32_t epilogue, void* workspace,
+                        int64_t workspace_bytes, void* stream);
 
 /*
  * The per-step bookkeeping of a captured CandidateGroup decode step (the
