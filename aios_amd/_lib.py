@@ -57,6 +57,8 @@ EXPORTED_SYMBOLS = (
     "aios_attnres_mix_ex",
     "aios_stateless_uniforms",
     "aios_sample",
+    "aios_sample_workspace",
+    "aios_sample_ws",
 )
 
 
@@ -184,6 +186,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.aios_sample.restype = ctypes.c_int
     lib.aios_sample.argtypes = [_vp, _i64, _i32, _i32, _i32, _f32, _i32, _f32, _vp, _i64, _i32,
                                 _vp, _vp, _i32, _i32, _vp, _i32, _vp, _vp, _vp]
+    lib.aios_sample_workspace.restype = _i64
+    lib.aios_sample_workspace.argtypes = [_i32, _i32, _f32, _i32, _f32]
+    lib.aios_sample_ws.restype = ctypes.c_int
+    lib.aios_sample_ws.argtypes = [_vp, _i64, _i32, _i32, _i32, _f32, _i32, _f32, _vp, _i64, _i32,
+                                   _vp, _vp, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _i64, _vp]
     lib.aios_attnres_mix.restype = ctypes.c_int
     lib.aios_attnres_mix.argtypes = [_vp, _i32, _i64, _i32, _vp, _vp, _f32, _vp, _vp, _vp]
     lib.aios_attnres_mix_ex.restype = ctypes.c_int

@@ -948,6 +948,26 @@ int aios_sample(const void* logits, int64_t row_stride, int32_t rows, int32_t vo
                 int32_t forbid_before_step, const int64_t* forbidden_by_row,
                 int32_t row_forbidden_count, int64_t* token_out, float* logprob_out,
                 void* stream) {
+  return aios_sample_ws(logits, row_stride, rows, vocab, elem_bytes, temperature, top_k, top_p,
+                        uniforms, uniform_stride, uniform_count, step, forbidden, n_forbidden,
+                        forbid_before_step, forbidden_by_row, row_forbidden_count, token_out,
+                        logprob_out, nullptr, 0, stream);
+}
+
+int64_t aios_sample_workspace(int32_t rows, int32_t vocab, float temperature, int32_t top_k,
+                              float top_p) {
+  if (rows <= 0 || vocab <= 0) return 0;
+  const bool greedy = (temperature <= 0.f || top_k == 1) && top_p == 1.f;
+  return aios::sample_workspace(rows, vocab, greedy ? 1 : top_k);
+}
+
+int aios_sample_ws(const void* logits, int64_t row_stride, int32_t rows, int32_t vocab,
+                   int32_t elem_bytes, float temperature, int32_t top_k, float top_p,
+                   const float* uniforms, int64_t uniform_stride, int32_t uniform_count,
+                   const int64_t* step, const int32_t* forbidden, int32_t n_forbidden,
+                   int32_t forbid_before_step, const int64_t* forbidden_by_row,
+                   int32_t row_forbidden_count, int64_t* token_out, float* logprob_out,
+                   void* workspace, int64_t workspace_bytes, void* stream) {
   if (rows < 0 || vocab <= 0 || (row_stride != 0 && row_stride < vocab))
     return fail(AIOS_ERR_INVALID, "sample: bad sizes (rows=%d vocab=%d stride=%lld)", rows, vocab,
                 (long long)row_stride);
@@ -996,7 +1016,10 @@ int aios_sample(const void* logits, int64_t row_stride, int32_t rows, int32_t vo
   a.row_forbidden_count = row_forbidden_count;
   a.token_out = token_out;
   a.logprob_out = logprob_out;
-  return check_hip(aios::sample_rows(a, static_cast<hipStream_t>(stream)), "sample launch");
+  const bool ws = ((uintptr_t)workspace & 15) == 0;
+  return check_hip(aios::sample_rows(a, ws ? workspace : nullptr, workspace_bytes,
+                                     static_cast<hipStream_t>(stream)),
+                   "sample launch");
 }
 
 static bool overlaps(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {

@@ -257,7 +257,10 @@ struct SampleArgs {
 };
 constexpr int kSampleMaxTopK = 1024;
 constexpr int kSampleMaxForbidden = 256;
-hipError_t sample_rows(const SampleArgs& a, hipStream_t stream);
+// Bytes of workspace with which long rows are split over workgroups (0: not).
+int64_t sample_workspace(int32_t rows, int32_t vocab, int32_t top_k);
+hipError_t sample_rows(const SampleArgs& a, void* workspace, int64_t workspace_bytes,
+                       hipStream_t stream);
 hipError_t stateless_uniforms(const int64_t* seeds, int32_t rows, int32_t steps, float* out,
                               hipStream_t stream);
 

@@ -1,8 +1,10 @@
 // Token selection with the raw log-probability of the chosen token:
 // greedy_kernel (argmax), and stateless temperature / top-k / top-p sampling
 // (python/aios/engine/sample.py:12-160) by sample_resident_kernel (top-k
-// over rows of at most 16384 ids, the row held in registers) or
-// sample_kernel (longer rows, and every id in id order, streaming the row).
+// over rows of at most 16384 ids, the row held in registers), by
+// sample_segment_kernel and sample_merge_kernel (top-k over longer rows, a
+// workgroup per segment, then one per row) or by sample_kernel (every id in
+// id order, and longer rows without a workspace, streaming the row).
 //
 // Greedy:
 // One workgroup per row.  token = the first index of the row maximum of the
@@ -810,13 +812,16 @@ struct ResKeyOf<float> {
 };
 static_assert(kResMaxVocab <= (1 << 16), "ids fit the 16-bit field of the bf16 keys");
 
-template <typename Key, int NW>
-struct ResShared {
+template <int NW>
+struct ResSelect {
   uint32_t fbits[kResMaxVocab / 32];   // forbidden ids, one bit each
   alignas(16) uint32_t red[2][NW][8];  // per-wavefront packed counts
   float fred[2][NW][2];                // per-wavefront max / sum
   uint32_t ired[2][NW];                // per-wavefront counts (bisection)
   uint32_t gscan[NW];                  // per-wavefront candidate counts
+};
+template <typename Key>
+struct ResOrder {
   alignas(16) Key cand[kResCap];
   Key top[kSampleMaxTopK];
   float ev[kSampleMaxTopK];  // exp of the top k (wavefront 0)
@@ -969,23 +974,32 @@ __device__ __forceinline__ float res_block_counts(const uint64_t (&acc)[NC], uin
   return ftot;
 }
 
-template <typename T, int NT, int NC>
-__global__ __launch_bounds__(NT) void sample_resident_kernel(SampleArgs a) {
+// The code of a distance below the maximum (see above).
+__device__ __forceinline__ uint32_t res_code(float d) {
+  const uint32_t eb = __float_as_uint(d) >> 19;
+  return min(eb - min(eb, 118u << 4), 254u);
+}
+
+struct ResSelected {
+  int n;             // candidates written
+  float rmax, rsum;  // raw maximum and sum of exp(x - rmax)
+};
+
+// Steps 1 to 3 and 5 over ids id0 .. id0 + vocab - 1 of row `row` (x at id0):
+// at least min(top_k, vocab) candidates, the top ones among them, as
+// composite keys in cand (LDS or global memory; at most kResCap).  The
+// writes to cand are not yet ordered for other threads.
+template <typename T, typename Key, int kIdBits, int NT, int NC>
+__device__ __forceinline__ ResSelected res_select(const SampleArgs& a, ResSelect<NT / 64>& sh, Key* cand,
+                                                  const T* x, int row, int id0, int vocab) {
   constexpr int NW = NT / 64;
   static_assert(NT * 8 * NC <= kResMaxVocab && kSampleMaxForbidden <= NT, "row and lists fit");
   static_assert(NC * 8 <= 32, "a thread's ids index 32-bit masks");
   using L = LogitTraits<T>;
-  using Key = typename ResKeyOf<T>::Key;
-  constexpr int kIdBits = ResKeyOf<T>::kIdBits;
   constexpr Key kIdMask = (Key)((1ull << kIdBits) - 1);
-  __shared__ ResShared<Key, NW> sh;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int row = blockIdx.x;
-  const int vocab = a.vocab;
-  const T* x = static_cast<const T*>(a.logits) + (int64_t)row * a.row_stride;
-  const uint32_t neg_key = L::key(L::kBits == 16 ? 0xff80u : 0xff800000u);
 
   // The row (chunk c of this thread: ids 8 (c * NT + tid) + j).
   float v[NC][8];
@@ -1002,15 +1016,13 @@ __global__ __launch_bounds__(NT) void sample_resident_kernel(SampleArgs a) {
   // step < forbid_before_step, then row r's list
   int fid = -1;
   if (tid < a.n_forbidden) {
-    const int32_t f = a.forbidden[tid];
-    fid = (step < a.forbid_before_step && f >= 0 && f < vocab) ? f : -1;
+    const int64_t f = (int64_t)a.forbidden[tid] - id0;
+    fid = (step < a.forbid_before_step && f >= 0 && f < vocab) ? (int)f : -1;
   } else if (tid < a.n_forbidden + a.row_forbidden_count) {
-    const int64_t f = a.forbidden_by_row[(int64_t)row * a.row_forbidden_count + tid - a.n_forbidden];
+    const int64_t f =
+        a.forbidden_by_row[(int64_t)row * a.row_forbidden_count + tid - a.n_forbidden] - id0;
     fid = (f >= 0 && f < vocab) ? (int)f : -1;
   }
-  const int64_t col = step < 0 ? 0 : (step >= a.uniform_count ? a.uniform_count - 1 : step);
-  const float u = a.uniforms != nullptr ? a.uniforms[(int64_t)row * a.uniform_stride + col] : 0.5f;
-
   // 1. forbidden bitmap
   for (int i = tid; i < (vocab + 31) / 32; i += NT) sh.fbits[i] = 0u;
   __syncthreads();
@@ -1048,8 +1060,7 @@ __global__ __launch_bounds__(NT) void sample_resident_kernel(SampleArgs a) {
       rs += fast_exp2(v[c][j] * kLog2e - mu);
       if ((fb >> j) & 1u) v[c][j] = kNegInf;
       const float d = rmax - v[c][j];  // +0 at the maximum; inf or NaN at -inf
-      const uint32_t eb = __float_as_uint(d) >> 19;
-      const uint32_t cb = min(eb - min(eb, 118u << 4), 254u);
+      const uint32_t cb = res_code(d);
       code[c][j >> 2] |= cb << (8 * (j & 3));
       acc[c] += 1ull << ((cb >> 4) * 4);
     }
@@ -1064,7 +1075,6 @@ __global__ __launch_bounds__(NT) void sample_resident_kernel(SampleArgs a) {
   const float rsum = res_block_counts<NC, NW>(acc, sh.red[0], sh.fred[1], rs, lane, wave, tot);
   const int n_pad_ids = NC * NT * 8 - vocab;  // ids past the row, all in bucket 15
   tot[15] -= n_pad_ids;
-  const float log_z = rmax + logf(rsum);
   const int k = min(a.top_k, vocab);
   int oct = 15, below = 0;
   {
@@ -1111,12 +1121,11 @@ __global__ __launch_bounds__(NT) void sample_resident_kernel(SampleArgs a) {
 
   auto id_of = [&](int c, int j) { return (c * NT + tid) * 8 + j; };
   auto ckey = [&](int c, int j) {
-    return ((Key)res_vkey(v[c][j], (T*)nullptr) << kIdBits) | (kIdMask - (Key)id_of(c, j));
+    return ((Key)res_vkey(v[c][j], (T*)nullptr) << kIdBits) | (kIdMask - (Key)(id0 + id_of(c, j)));
   };
-  // Writes the ids for which pred(c, j) holds to sh.cand (wavefront by
+  // Writes the ids for which pred(c, j) holds to cand (wavefront by
   // wavefront, id slot by id slot: one ballot per slot, positions from the
-  // wavefront totals and mbcnt) and zero keys after them up to the next
-  // power of two; returns how many.
+  // wavefront totals and mbcnt); returns how many.
   auto gather = [&](auto&& pred) -> int {
     uint32_t wcnt = 0u;
 #pragma unroll
@@ -1141,16 +1150,11 @@ __global__ __launch_bounds__(NT) void sample_resident_kernel(SampleArgs a) {
         if (mk != 0ull) {
           const uint32_t at = pos + __builtin_amdgcn_mbcnt_hi(
                                         (uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0u));
-          if (pr && at < (uint32_t)kResCap) sh.cand[at] = ckey(c, j);
+          if (pr && at < (uint32_t)kResCap) cand[at] = ckey(c, j);
           pos += __popcll(mk);
         }
       }
-    const int cnt = (int)min(total, (uint32_t)kResCap);
-    int npad = 1;
-    while (npad < cnt) npad <<= 1;
-    for (int i = cnt + tid; i < npad; i += NT) sh.cand[i] = 0;
-    __syncthreads();
-    return cnt;
+    return (int)min(total, (uint32_t)kResCap);
   };
 
   auto in_row = [&](int c, int j) { return ((valid >> (8 * c + j)) & 1u) != 0u; };
@@ -1212,11 +1216,27 @@ __global__ __launch_bounds__(NT) void sample_resident_kernel(SampleArgs a) {
       });
     }
   }
+  return ResSelected{n, rmax, rsum};
+}
 
-  // 4. order the candidates; the first k go to sh.top
-  // (the gather left zero keys, below every real key, up to npad)
+// Steps 4 and 6: the id picked from the n >= k candidates in sh.cand (not
+// necessarily ordered for this thread yet) with uniform u, and its raw
+// log-probability, stored for row `row` (x: its logits).
+template <typename T, typename Key, int kIdBits, int NT>
+__device__ __forceinline__ void res_pick(const SampleArgs& a, ResOrder<Key>& sh, const T* x, int row, int n,
+                                         int k, float u, float log_z) {
+  using L = LogitTraits<T>;
+  constexpr Key kIdMask = (Key)((1ull << kIdBits) - 1);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const uint32_t neg_key = L::key(L::kBits == 16 ? 0xff80u : 0xff800000u);
+  // 4. order the candidates; the first k go to sh.top (zero keys, below every
+  // real key, up to npad)
   int npad = 1;
   while (npad < n) npad <<= 1;
+  for (int i = n + tid; i < npad; i += NT) sh.cand[i] = 0;
+  __syncthreads();
   if (n <= kResRankMax) {
     // tpe threads per candidate, each counting the larger keys in its own
     // contiguous run of L entries
@@ -1320,6 +1340,162 @@ __global__ __launch_bounds__(NT) void sample_resident_kernel(SampleArgs a) {
   }
 }
 
+// The step's uniform of row `row` (the step clamped into the table).
+__device__ __forceinline__ float res_uniform(const SampleArgs& a, int row) {
+  const int64_t step = a.step != nullptr ? *a.step : 0;
+  const int64_t col = step < 0 ? 0 : (step >= a.uniform_count ? a.uniform_count - 1 : step);
+  return a.uniforms != nullptr ? a.uniforms[(int64_t)row * a.uniform_stride + col] : 0.5f;
+}
+
+template <typename T, int NT, int NC>
+__global__ __launch_bounds__(NT) void sample_resident_kernel(SampleArgs a) {
+  using Key = typename ResKeyOf<T>::Key;
+  constexpr int kIdBits = ResKeyOf<T>::kIdBits;
+  __shared__ ResSelect<NT / 64> sel;
+  __shared__ ResOrder<Key> ord;
+  const int row = blockIdx.x;
+  const T* x = static_cast<const T*>(a.logits) + (int64_t)row * a.row_stride;
+  const float u = res_uniform(a, row);
+  const ResSelected r = res_select<T, Key, kIdBits, NT, NC>(a, sel, ord.cand, x, row, 0, a.vocab);
+  res_pick<T, Key, kIdBits, NT>(a, ord, x, row, r.n, min(a.top_k, a.vocab), u, r.rmax + logf(r.rsum));
+}
+
+// Longer rows, top_k >= 1: the row's segments of kSegIds ids are selected by
+// a workgroup each (sample_segment_kernel: the resident kernel's steps up to
+// the candidates, written to global memory with the segment's raw maximum
+// and sum of exp), then one workgroup per row merges (sample_merge_kernel):
+// every segment's top k are among its candidates, so the row's are among all
+// of them; a count of their codes (distance below the row's maximum, as in
+// the resident kernel) over 256 LDS bins finds an upper set of at least k,
+// which is ordered and sampled as there.  One workgroup per row alone took
+// 376 us for 24 bf16 rows of 151,936 ids, top_k 50 (sample_kernel: three sweeps
+// of one compute unit with up to 16 compares per id);
+// split, 12.1 us for the segments and 6.8 us for the merge.
+constexpr int kSegThreads = 512;
+constexpr int kSegIds = 8192;
+constexpr int kMaxSegs = 64;          // segments of a row (one lane each in the merge)
+constexpr int kMergeStage = 4096;     // candidates the merge keeps in LDS
+constexpr int64_t kSegMaxBytes = 256ll << 20;  // more rows than this takes fill the chip by themselves
+
+struct SegHead {
+  int32_t n;
+  float rmax, rsum;
+  int32_t unused;
+};
+using SegKey = unsigned long long;  // value key << 32 | (0xffffffff - id)
+
+template <typename T>
+__global__ __launch_bounds__(kSegThreads) void sample_segment_kernel(SampleArgs a, int32_t segs,
+                                                                     SegHead* heads, SegKey* cand) {
+  __shared__ ResSelect<kSegThreads / 64> sel;
+  const int row = blockIdx.x / segs;
+  const int seg = blockIdx.x - row * segs;
+  const int id0 = seg * kSegIds;
+  const T* x = static_cast<const T*>(a.logits) + (int64_t)row * a.row_stride + id0;
+  const ResSelected r = res_select<T, SegKey, 32, kSegThreads, kSegIds / (8 * kSegThreads)>(
+      a, sel, cand + (int64_t)blockIdx.x * kResCap, x, row, id0, min(a.vocab - id0, kSegIds));
+  if (threadIdx.x == 0) heads[blockIdx.x] = SegHead{r.n, r.rmax, r.rsum, 0};
+}
+
+template <typename T>
+__global__ __launch_bounds__(kSegThreads) void sample_merge_kernel(SampleArgs a, int32_t segs,
+                                                                   const SegHead* heads,
+                                                                   const SegKey* cand) {
+  using L = LogitTraits<T>;
+  constexpr int NW = kSegThreads / 64;
+  __shared__ ResOrder<SegKey> ord;
+  __shared__ SegKey stage[kMergeStage];
+  __shared__ alignas(16) uint32_t hist[256];
+  __shared__ uint32_t count[2];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = blockIdx.x;
+  const T* x = static_cast<const T*>(a.logits) + (int64_t)row * a.row_stride;
+  const float u = res_uniform(a, row);
+  const int k = min(a.top_k, a.vocab);
+  heads += (int64_t)row * segs;
+  cand += (int64_t)row * segs * kResCap;
+  // lane s: segment s
+  const SegHead h = lane < segs ? heads[lane] : SegHead{0, kNegInf, 0.f, 0};
+  if (tid < 256) hist[tid] = 0u;
+  if (tid < 2) count[tid] = 0u;
+  const float rmax = lanes_max_f(h.rmax);
+  const float rsum =
+      lanes_sum_f(h.rmax == kNegInf ? 0.f : h.rsum * fast_exp2((h.rmax - rmax) * kLog2e));
+  const uint32_t ends = lanes_scan_u((uint32_t)h.n);
+  const int total = (int)__builtin_amdgcn_readlane(ends, 63);
+  const bool staged = total <= kMergeStage;
+  __syncthreads();
+  // Every candidate of the row once: f(key, index over the row).
+  auto sweep = [&](auto&& f) {
+    for (int s = wave; s < segs; s += NW) {
+      const int n = __builtin_amdgcn_readlane(h.n, s);
+      const int at = (int)__builtin_amdgcn_readlane(ends, s) - n;
+      for (int i0 = 0; i0 < n; i0 += 256) {
+        SegKey key[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          key[q] = cand[(int64_t)s * kResCap + min(i0 + q * 64 + lane, n - 1)];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (i0 + q * 64 + lane < n) f(key[q], at + i0 + q * 64 + lane);
+      }
+    }
+  };
+  auto code = [&](SegKey key) { return res_code(rmax - L::value((uint32_t)(key >> 32))); };
+  sweep([&](SegKey key, int i) {
+    if (staged) stage[i] = key;
+    atomicAdd(&hist[code(key)], 1u);
+  });
+  __syncthreads();
+  // The smallest code whose cumulative count reaches k (lane l: bins 4 l ..).
+  const uint4 hb = reinterpret_cast<const uint4*>(hist)[lane];
+  const uint32_t below = lanes_scan_u(hb.x + hb.y + hb.z + hb.w) - (hb.x + hb.y + hb.z + hb.w);
+  const uint32_t c0 = below + hb.x, c1 = c0 + hb.y, c2 = c1 + hb.z, c3 = c2 + hb.w;
+  const uint32_t kk = (uint32_t)k;
+  const uint64_t has = __ballot(c3 >= kk);  // (never empty: the candidates number at least k)
+  const int first = has ? __builtin_ctzll(has) : 63;
+  const int in4 = c0 >= kk ? 0 : c1 >= kk ? 1 : c2 >= kk ? 2 : 3;
+  const uint32_t bound = (uint32_t)(first * 4 + __builtin_amdgcn_readlane(in4, first));
+  const uint32_t c4 = in4 == 0 ? c0 : in4 == 1 ? c1 : in4 == 2 ? c2 : c3;
+  int n = (int)__builtin_amdgcn_readlane(c4, first);
+  auto gather = [&](auto&& pred) {
+    auto take = [&](SegKey key, int) {
+      if (pred(key)) ord.cand[atomicAdd(&count[0], 1u)] = key;
+    };
+    if (staged) {
+      for (int i = tid; i < total; i += kSegThreads) take(stage[i], i);
+    } else {
+      sweep(take);
+    }
+  };
+  if (n <= kResCap) {
+    gather([&](SegKey key) { return code(key) <= bound; });
+  } else {
+    // Ids tied within the bound's code overflow the buffer: the k-th largest
+    // composite key (they are distinct) by bisection, exactly the top k.
+    SegKey lo = 0, hi = ~0ull;
+    while (lo < hi) {
+      const SegKey mid = lo + ((hi - lo) >> 1) + 1;
+      uint32_t cnt = 0u;
+      sweep([&](SegKey key, int) { cnt += key >= mid ? 1u : 0u; });
+      cnt = lanes_sum_u(cnt);
+      if (lane == 0) atomicAdd(&count[1], cnt);
+      __syncthreads();
+      const uint32_t c = count[1];
+      __syncthreads();
+      if (tid == 0) count[1] = 0u;
+      __syncthreads();
+      if (c >= kk) lo = mid;
+      else hi = mid - 1;
+    }
+    n = k;
+    gather([&](SegKey key) { return key >= lo; });
+  }
+  res_pick<T, SegKey, 32, kSegThreads>(a, ord, x, row, n, k, u, rmax + logf(rsum));
+}
+
 // One uniform per (row, step): SplitMix64 of seed + (step + 1) * golden
 // ratio, 53 high bits + 0.5 over 2^53, rounded to fp32 (sample.py:12-47).
 __global__ void uniforms_kernel(const int64_t* __restrict__ seeds, int32_t rows, int32_t steps,
@@ -1350,11 +1526,31 @@ static void launch_resident(const SampleArgs& a, hipStream_t stream) {
     sample_resident_kernel<T, NT, kResMaxVocab / (NT * 8)><<<grid, block, 0, stream>>>(a);
 }
 
-hipError_t sample_rows(const SampleArgs& a, hipStream_t stream) {
+// Workspace of the split form: segment heads, then candidate keys.
+int64_t sample_workspace(int32_t rows, int32_t vocab, int32_t top_k) {
+  const int64_t segs = ((int64_t)vocab + kSegIds - 1) / kSegIds;
+  if (top_k < 1 || vocab <= kResMaxVocab || segs > kMaxSegs) return 0;
+  const int64_t bytes = rows * segs * ((int64_t)sizeof(SegHead) + kResCap * (int64_t)sizeof(SegKey));
+  return bytes <= kSegMaxBytes ? bytes : 0;
+}
+
+template <typename T>
+static hipError_t launch_segments(const SampleArgs& a, void* workspace, hipStream_t stream) {
+  const int32_t segs = (a.vocab + kSegIds - 1) / kSegIds;
+  SegHead* heads = static_cast<SegHead*>(workspace);
+  SegKey* cand = reinterpret_cast<SegKey*>(heads + (int64_t)a.rows * segs);
+  sample_segment_kernel<T><<<dim3(a.rows * segs), dim3(kSegThreads), 0, stream>>>(a, segs, heads, cand);
+  sample_merge_kernel<T><<<dim3(a.rows), dim3(kSegThreads), 0, stream>>>(a, segs, heads, cand);
+  return hipGetLastError();
+}
+
+hipError_t sample_rows(const SampleArgs& a, void* workspace, int64_t workspace_bytes,
+                       hipStream_t stream) {
   if (a.rows == 0) return hipSuccess;
   // top-k (greedy included) over a row that fits the registers of one
-  // workgroup: the row-resident kernel; every id in id order (top_k 0) and
-  // longer rows: the streaming kernel
+  // workgroup: the row-resident kernel; longer rows: in segments, given room
+  // for their candidates; every id in id order (top_k 0), and longer rows
+  // without that room: the streaming kernel
   if (a.top_k >= 1 && a.vocab <= kResMaxVocab) {
     if (a.elem_bytes == 2)
       launch_resident<bf16>(a, stream);
@@ -1362,6 +1558,10 @@ hipError_t sample_rows(const SampleArgs& a, hipStream_t stream) {
       launch_resident<float>(a, stream);
     return hipGetLastError();
   }
+  const int64_t need = sample_workspace(a.rows, a.vocab, a.top_k);
+  if (need > 0 && workspace != nullptr && workspace_bytes >= need)
+    return a.elem_bytes == 2 ? launch_segments<bf16>(a, workspace, stream)
+                             : launch_segments<float>(a, workspace, stream);
   if (a.elem_bytes == 2)
     sample_kernel<bf16><<<dim3(a.rows), dim3(kSampleThreads), 0, stream>>>(a);
   else

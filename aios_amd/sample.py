@@ -5,7 +5,7 @@ python/aios/engine/sample.py: ``stateless_uniforms`` and
 ``stateless_uniforms`` computes the SplitMix64 uniforms on the device
 (``aios_stateless_uniforms``), keyed by (candidate seed, token step), so a
 candidate keeps its stream wherever its row sits in the batch.
-``Sampler.sample_with_logprobs`` is one launch of ``aios_sample`` per call:
+``Sampler.sample_with_logprobs`` is one call of ``aios_sample_ws``:
 temperature / top-k / top-p on a sampling copy with forbidden ids at -inf,
 the token chosen by the candidate's uniform, and the raw log-probability of
 the unmodified distribution.  ``sample_step`` is the same launch with the
@@ -83,13 +83,19 @@ def sample_step(logits: torch.Tensor, params: SamplingParams, uniforms: torch.Te
         torch.empty(rows, dtype=torch.float32, device=logits.device))
     nf = 0 if forbidden_ids is None else forbidden_ids.numel()
     nr = 0 if forbidden_by_row is None else forbidden_by_row.shape[1]
-    _lib.check(_lib.lib().aios_sample(
+    lib = _lib.lib()
+    # (the candidates of long rows: a buffer of this call alone, since calls may
+    # overlap on several streams)
+    ws_bytes = lib.aios_sample_workspace(rows, vocab, float(params.temperature),
+                                         int(params.top_k), float(params.top_p))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=logits.device) if ws_bytes else None
+    _lib.check(lib.aios_sample_ws(
         logits.data_ptr(), logits.stride(0), rows, vocab, logits.element_size(),
         float(params.temperature), int(params.top_k), float(params.top_p),
         uniforms.data_ptr(), uniforms.stride(0), uniforms.shape[1], step.data_ptr(),
         forbidden_ids.data_ptr() if nf else None, nf, int(forbid_before_step),
         forbidden_by_row.data_ptr() if nr else None, nr, tok.data_ptr(), lp.data_ptr(),
-        _stream(logits)), "aios_sample")
+        ws.data_ptr() if ws is not None else None, ws_bytes, _stream(logits)), "aios_sample_ws")
     return tok, lp
 
 

@@ -489,6 +489,21 @@ int aios_sample(const void* logits, int64_t row_stride, int32_t rows, int32_t vo
                 void* stream);
 
 /*
+ * aios_sample with a 16-byte aligned workspace: long rows are split over
+ * workgroups when it holds the aios_sample_workspace(...) bytes (0: none
+ * used; a smaller or null workspace runs one workgroup per row).
+ */
+int64_t aios_sample_workspace(int32_t rows, int32_t vocab, float temperature, int32_t top_k,
+                              float top_p);
+int aios_sample_ws(const void* logits, int64_t row_stride, int32_t rows, int32_t vocab,
+                   int32_t elem_bytes, float temperature, int32_t top_k, float top_p,
+                   const float* uniforms, int64_t uniform_stride, int32_t uniform_count,
+                   const int64_t* step, const int32_t* forbidden, int32_t n_forbidden,
+                   int32_t forbid_before_step, const int64_t* forbidden_by_row,
+                   int32_t row_forbidden_count, int64_t* token_out, float* logprob_out,
+                   void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Block-AttnRes depth mix.  bank is contiguous bf16 [bank_sources]
  * [num_tokens][hidden]; partial (may be NULL) a contiguous bf16
  * [num_tokens][hidden] plane appended as the last source;

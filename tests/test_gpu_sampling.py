@@ -241,3 +241,47 @@ def test_sample_rejects_unsupported():
     with pytest.raises(ValueError, match="uniforms must match"):
         Sampler(SamplingParams(temperature=1.0, top_k=5)).sample_with_logprobs(
             x, uniforms=torch.full((3,), 0.5, device="cuda"))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [16385, 24577, 65544, 151936])
+def test_sample_split_rows(dtype, vocab):
+    """Rows split into 8192-id segments (a last segment of one id, of eight):
+    top ids in one segment or in all, ids forbidden in several segments, and
+    rows whose finite ids number fewer than top_k."""
+    rows = 6
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    stride = (vocab + 7) // 8 * 8
+    full = (torch.randn(rows, stride, generator=g, device="cuda") * 2.0).to(dtype)
+    x = full[:, :vocab]
+    x[0, 8192:8292] += 12.0           # the whole top k in the second segment
+    x[1, :: max(1, vocab // 60)] += 9.0  # spread over all segments
+    x[2, 100:] = -float("inf")
+    x[3, : vocab - 1] = -float("inf")  # a single finite id, the last
+    x[4, vocab - 1] = 30.0             # the last id dominates
+    u = stateless_uniforms([9 * vocab + r for r in range(rows)], 1, torch.device("cuda"))[:, 0]
+    by_row = torch.tensor([[8200, 16384], [0, vocab - 2], [5, 6], [7, 8192], [1, vocab - 1],
+                           [3, 3]], dtype=torch.int64, device="cuda")
+    for params in (SamplingParams(temperature=0.35, top_k=50, top_p=0.9),
+                   SamplingParams(temperature=1.0, top_k=700, top_p=1.0),
+                   SamplingParams(temperature=0.0)):
+        _check_rows(x, params, u)
+        _check_rows(x, params, u, forbidden=(2, 8193), by_row=by_row)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_sample_split_rows_tied_beyond_the_candidate_buffer(dtype):
+    """Four distinct values over 151,936 ids: every segment's candidates are the
+    lowest of its ties, and the row's overflow the merge's buffer too, so the
+    cut among them is found by bisection on (value, id)."""
+    rows, vocab = 4, 151936
+    g = torch.Generator(device="cuda").manual_seed(12)
+    x = (torch.randint(0, 4, (rows, vocab), generator=g, device="cuda").to(torch.float32) * 0.5).to(dtype)
+    u = stateless_uniforms([50 + r for r in range(rows)], 1, torch.device("cuda"))[:, 0]
+    top = [int((x[r].float() == 1.5).nonzero()[0].item()) for r in range(rows)]
+    by_row = torch.tensor([[t, t + 1] for t in top], dtype=torch.int64, device="cuda")
+    for params in (SamplingParams(temperature=0.5, top_k=50, top_p=0.9),
+                   SamplingParams(temperature=1.0, top_k=1024, top_p=1.0),
+                   SamplingParams(temperature=0.0)):
+        _check_rows(x, params, u)
+        _check_rows(x, params, u, forbidden=(3,), by_row=by_row)
