@@ -44,6 +44,7 @@ EXPORTED_SYMBOLS = (
     "aios_rmsnorm",
     "aios_add_rmsnorm",
     "aios_qk_norm_rope",
+    "aios_qk_norm_rope_append",
     "aios_cg_step_begin",
     "aios_cg_step_end",
     "aios_cg_step_prepare",
@@ -97,6 +98,15 @@ class AttnPlan(ctypes.Structure):
 
     def as_dict(self) -> dict:
         return {name: getattr(self, name) for name, _ in self._fields_}
+
+
+def raw_stream(device) -> int:
+    """The current HIP stream handle of a torch GPU device (the handle alone:
+    torch.cuda.current_stream builds a Stream object, 2 us of each launch)."""
+    import torch
+
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 _lock = threading.Lock()
@@ -164,6 +174,9 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.aios_cg_step_end.restype = ctypes.c_int
     lib.aios_cg_step_end.argtypes = [_vp, _i32, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _i32, _vp,
                                      _vp, _vp, _vp, _vp, _vp]
+    lib.aios_qk_norm_rope_append.restype = ctypes.c_int
+    lib.aios_qk_norm_rope_append.argtypes = [_vp, _i64, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp,
+                                             _i64, _vp, _vp, _vp, _vp, _i64, _vp, _f32, _vp]
     lib.aios_qk_norm_rope.restype = ctypes.c_int
     lib.aios_qk_norm_rope.argtypes = [_vp, _i64, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64,
                                       _vp, _vp, _vp, _f32, _vp]

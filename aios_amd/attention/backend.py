@@ -37,12 +37,12 @@ import torch
 
 from aios_amd import _lib, paged
 from aios_amd.core import get_global_ctx
+from aios_amd.kvcache import MHAKVCache
 
 from .base import BaseAttentionBackend, BaseAttentionMetadata
 
 if TYPE_CHECKING:
     from aios_amd.core import Batch
-    from aios_amd.kvcache import MHAKVCache
 
 SUPPORTED_HEAD_DIMS = frozenset({64, 96, 128})
 SUPPORTED_GROUPS = frozenset({1, 2, 3, 4, 6, 8})
@@ -488,9 +488,38 @@ class Mi355xAttentionBackend(BaseAttentionBackend):
         if q.shape[0] != metadata.plan.total_q:
             raise RuntimeError("prefill request lengths do not match flat Q tokens")
         paged_kv_cache.store_kv(k, v, batch.out_loc.view(-1), layer_id)
+        return self.prefill_appended(q, *self.layer_kv(paged_kv_cache, layer_id), batch)
+
+    def append_rope_applies(self, qkv: torch.Tensor, paged_kv_cache, batch: Batch) -> bool:
+        """Whether the K/V rows of this batch may be written by the launch that
+        normalises and rotates them (then layer_kv and prefill_appended run
+        the rest): a prefill batch with one int32 slot per row of qkv into a
+        pool of this package, whose store_kv that launch stands for.  Other
+        batches go through store_kv, with its conversions and errors."""
+        if not batch.is_prefill or not isinstance(batch.attn_metadata, Mi355xAttentionMetadata):
+            return False
+        if (type(self).forward is not Mi355xAttentionBackend.forward or "forward" in vars(self)
+                or type(paged_kv_cache).store_kv is not MHAKVCache.store_kv
+                or "store_kv" in vars(paged_kv_cache)):
+            return False  # (a caller's own forward or store_kv sees every call)
+        loc = batch.out_loc
+        return (paged_kv_cache.row_shape == (self.num_kv_heads, self.head_dim)
+                and paged_kv_cache.dtype == torch.bfloat16 and qkv.dtype == torch.bfloat16
+                and loc.dtype == torch.int32 and loc.is_contiguous() and loc.is_cuda
+                and loc.numel() == qkv.shape[0] == batch.attn_metadata.plan.total_q)
+
+    def layer_kv(self, paged_kv_cache, layer_id: int) -> tuple[torch.Tensor, torch.Tensor]:
+        """One layer's K and V caches as [pages, Hkv, D]."""
         k_cache, v_cache = self._layer_caches(paged_kv_cache, layer_id)
-        out = paged.prefill(metadata.plan, q, k_cache.view(-1, self.num_kv_heads, self.head_dim),
-                            v_cache.view(-1, self.num_kv_heads, self.head_dim), metadata.indices,
+        shape = (-1, self.num_kv_heads, self.head_dim)
+        return k_cache.view(shape), v_cache.view(shape)
+
+    def prefill_appended(self, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                         batch: Batch) -> torch.Tensor:
+        """The prefill of a batch whose K/V rows are in their pages of one
+        layer's caches (layer_kv)."""
+        metadata = batch.attn_metadata
+        out = paged.prefill(metadata.plan, q, k_cache, v_cache, metadata.indices,
                             metadata.cu_seqlens_q_gpu, metadata.cu_seqlens_k_gpu,
                             sm_scale=self.sm_scale)
         return out.reshape(q.size(0), -1)

@@ -123,8 +123,8 @@ void plan_prefill_parts(aios_attn_plan_t* p, const int32_t* cu_q, const int32_t*
   }
   const int32_t n = cdiv(longest, part_sub);
   const int64_t parts = (int64_t)p->batch_size * p->num_q_tiles * hkv * n;
-  const int64_t o_bytes = parts * aios::kPrefillRows * p->head_dim * 4;
-  const int64_t bytes = n > 1 ? o_bytes + align_up(parts * aios::kPrefillRows * 8, 256) : 0;
+  const int64_t o_bytes = align_up(parts * rows * p->head_dim * 4, 256);
+  const int64_t bytes = n > 1 ? o_bytes + align_up(parts * rows * 8, 256) : 0;
   if (bytes > ws_bytes || parts > 0x3fffffff) return;
   p->prefix_chunk_len = part_sub * 32;
   p->num_parts = n;
@@ -370,9 +370,8 @@ int aios_attn_prefill_ws(const aios_attn_plan_t* p, const void* q, int64_t q_tok
     a.n_parts = p->num_parts;
     a.part_o = reinterpret_cast<float*>(ws + p->ws_parts_o);
     a.part_ml = reinterpret_cast<float2*>(ws + p->ws_parts_lse);
-    const int32_t tok = p->max_q_len < a.q_tile ? p->max_q_len : a.q_tile;
-    return check_hip(aios::launch_prefill_split(D, a, tok * a.group,
-                                                static_cast<hipStream_t>(stream)),
+    a.part_rows = (p->max_q_len < a.q_tile ? p->max_q_len : a.q_tile) * a.group;
+    return check_hip(aios::launch_prefill_split(D, a, static_cast<hipStream_t>(stream)),
                      "prefill launch");
   }
   return check_hip(aios::launch_prefill(D, 4, a, p->num_q_tiles, p->batch_size,
@@ -683,9 +682,35 @@ int aios_qk_norm_rope(const void* qkv, int64_t qkv_stride, int64_t tokens, int32
     return fail(AIOS_ERR_INVALID, "qk_norm_rope: rows must be 4-byte aligned");
   return check_hip(aios::qk_norm_rope(qkv, qkv_stride, tokens, num_qo_heads, num_kv_heads, head_dim,
                                       q_weight, k_weight, cos_table, sin_table, table_rows,
-                                      positions, q_out, k_out, eps,
+                                      positions, q_out, k_out, eps, nullptr, 0, nullptr,
                                       static_cast<hipStream_t>(stream)),
                    "qk_norm_rope launch");
+}
+
+int aios_qk_norm_rope_append(const void* qkv, int64_t qkv_stride, int64_t tokens,
+                             int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,
+                             const void* q_weight, const void* k_weight, const float* cos_table,
+                             const float* sin_table, int64_t table_rows, const int32_t* positions,
+                             void* q_out, void* k_cache, void* v_cache, int64_t num_slots,
+                             const int32_t* out_loc, float eps, void* stream) {
+  if (tokens < 0 || num_qo_heads <= 0 || num_kv_heads <= 0 || table_rows <= 0 || num_slots < 0)
+    return fail(AIOS_ERR_INVALID, "qk_norm_rope_append: bad sizes");
+  if (!aios::head_dim_supported(head_dim))
+    return fail(AIOS_ERR_UNSUPPORTED, "qk_norm_rope_append: head_dim %d is not built", head_dim);
+  if (qkv_stride < (int64_t)(num_qo_heads + 2 * num_kv_heads) * head_dim || qkv_stride % 2 != 0)
+    return fail(AIOS_ERR_INVALID, "qk_norm_rope_append: qkv row stride too small");
+  if (tokens == 0) return AIOS_OK;
+  if (!qkv || !q_weight || !k_weight || !cos_table || !sin_table || !positions || !q_out ||
+      !k_cache || !v_cache || !out_loc)
+    return fail(AIOS_ERR_INVALID, "qk_norm_rope_append: null pointer");
+  if ((((uintptr_t)qkv | (uintptr_t)q_weight | (uintptr_t)k_weight | (uintptr_t)k_cache |
+        (uintptr_t)v_cache) & 3) != 0)
+    return fail(AIOS_ERR_INVALID, "qk_norm_rope_append: rows must be 4-byte aligned");
+  return check_hip(aios::qk_norm_rope(qkv, qkv_stride, tokens, num_qo_heads, num_kv_heads, head_dim,
+                                      q_weight, k_weight, cos_table, sin_table, table_rows,
+                                      positions, q_out, k_cache, eps, v_cache, num_slots, out_loc,
+                                      static_cast<hipStream_t>(stream)),
+                   "qk_norm_rope_append launch");
 }
 
 int aios_silu_mul(const void* x, int64_t x_stride, int64_t rows, int32_t intermediate, void* out,

@@ -94,8 +94,8 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
 
 // Dims 8 dg .. 8 dg + 7 of row m in a part's o.
 template <int D>
-__device__ __forceinline__ int64_t prefill_part_o(int64_t part, int dg, int m) {
-  return ((part * (D / 8) + dg) * kPrefillRows + m) * 8;
+__device__ __forceinline__ int64_t prefill_part_o(const PrefillArgs& a, int64_t part, int dg, int m) {
+  return ((part * (D / 8) + dg) * a.part_rows + m) * 8;
 }
 
 template <int D>
@@ -172,10 +172,10 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
     for (int nt = 0; nt < D / 32; ++nt)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        *reinterpret_cast<f32x4*>(a.part_o + prefill_part_o<D>(part, nt * 4 + j, m) + 4 * hl) =
+        *reinterpret_cast<f32x4*>(a.part_o + prefill_part_o<D>(a, part, nt * 4 + j, m) + 4 * hl) =
             f32x4{eng.o[nt][4 * j], eng.o[nt][4 * j + 1], eng.o[nt][4 * j + 2],
                   eng.o[nt][4 * j + 3]};
-    if (hl == 0) a.part_ml[part * kPrefillRows + m] = make_float2(eng.m_run, eng.l_run);
+    if (hl == 0) a.part_ml[part * a.part_rows + m] = make_float2(eng.m_run, eng.l_run);
     return;
   }
 
@@ -243,10 +243,10 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
           make_uint4(pack_bf16x2(acc0[0], acc0[1]), pack_bf16x2(acc0[2], acc0[3]),
                      pack_bf16x2(acc1[0], acc1[1]), pack_bf16x2(acc1[2], acc1[3]));
     } else {
-      f32x4* po = reinterpret_cast<f32x4*>(a.part_o + prefill_part_o<D>(part, dg, row));
+      f32x4* po = reinterpret_cast<f32x4*>(a.part_o + prefill_part_o<D>(a, part, dg, row));
       po[0] = acc0;
       po[1] = acc1;
-      if (dg == 0) a.part_ml[part * kPrefillRows + row] = make_float2(mx, l);
+      if (dg == 0) a.part_ml[part * a.part_rows + row] = make_float2(mx, l);
     }
   }
 }
@@ -283,9 +283,9 @@ __global__ __launch_bounds__(NW * 64) void prefill_combine_kernel(PrefillArgs a,
   const bool ok = lane < RB * DG && m < rows;
   const int64_t part0 = (((int64_t)r * a.q_tiles + qt) * a.num_kv_heads + h) * a.n_parts;
   const f32x4* po =
-      reinterpret_cast<const f32x4*>(a.part_o + prefill_part_o<D>(part0, dg, ok ? m : 0));
-  constexpr int64_t kPartStride = (int64_t)D * kPrefillRows / 4;
-  const float2* ml = a.part_ml + part0 * kPrefillRows + (ok ? m : 0);
+      reinterpret_cast<const f32x4*>(a.part_o + prefill_part_o<D>(a, part0, dg, ok ? m : 0));
+  const int64_t part_stride = (int64_t)D / 4 * a.part_rows;
+  const float2* ml = a.part_ml + part0 * a.part_rows + (ok ? m : 0);
   float mx = kNegInf, l = 0.f;
   f32x4 acc0 = f32x4{0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
   for (int j0 = wave; j0 < pp.n; j0 += NW * NB) {
@@ -295,9 +295,9 @@ __global__ __launch_bounds__(NW * 64) void prefill_combine_kernel(PrefillArgs a,
     for (int k = 0; k < NB; ++k) {
       const int j = j0 + k * NW;
       if (j < pp.n) {  // (uniform per wavefront)
-        w[k] = ml[(int64_t)j * kPrefillRows];
-        x0[k] = po[j * kPartStride];
-        x1[k] = po[j * kPartStride + 1];
+        w[k] = ml[(int64_t)j * a.part_rows];
+        x0[k] = po[j * part_stride];
+        x1[k] = po[j * part_stride + 1];
       } else {
         w[k] = make_float2(kNegInf, 0.f);
         x0[k] = x1[k] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -354,14 +354,14 @@ __global__ __launch_bounds__(NW * 64) void prefill_combine_kernel(PrefillArgs a,
 }
 
 template <int D>
-static hipError_t launch_split_d(const PrefillArgs& a, int rows_max, hipStream_t s) {
+static hipError_t launch_split_d(const PrefillArgs& a, hipStream_t s) {
   const int tiles = a.q_tiles * a.num_kv_heads * a.batch;
   if (tiles == 0) return hipSuccess;
   hipLaunchKernelGGL(prefill_split_kernel<D>, dim3(tiles * a.n_parts), dim3(kEngineThreads), 0, s,
                      a);
   if (a.n_parts > 1) {
     constexpr int RB = 64 / (D / 8);
-    const int row_blocks = (rows_max + RB - 1) / RB;
+    const int row_blocks = (a.part_rows + RB - 1) / RB;
     const dim3 grid(tiles * row_blocks);
     if (a.n_parts <= 4)
       hipLaunchKernelGGL((prefill_combine_kernel<D, 1, 4>), grid, dim3(64), 0, s, a, row_blocks);
@@ -371,11 +371,11 @@ static hipError_t launch_split_d(const PrefillArgs& a, int rows_max, hipStream_t
   return hipGetLastError();
 }
 
-hipError_t launch_prefill_split(int D, const PrefillArgs& a, int rows_max, hipStream_t s) {
+hipError_t launch_prefill_split(int D, const PrefillArgs& a, hipStream_t s) {
   switch (D) {
-    case 64: return launch_split_d<64>(a, rows_max, s);
-    case 96: return launch_split_d<96>(a, rows_max, s);
-    case 128: return launch_split_d<128>(a, rows_max, s);
+    case 64: return launch_split_d<64>(a, s);
+    case 96: return launch_split_d<96>(a, s);
+    case 128: return launch_split_d<128>(a, s);
     default: return hipErrorInvalidValue;
   }
 }

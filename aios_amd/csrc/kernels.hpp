@@ -107,16 +107,16 @@ struct PrefillArgs {
   // The partial states of tile slot t = (r * q_tiles + qt) * Hkv + h, part s
   // (s < the tile's own part count), all fp32 and relative to the row's
   // reference m:
-  //   part_o  [slots][n_parts][D / 8][kPrefillRows][8]  unnormalised o
-  //   part_ml [slots][n_parts][kPrefillRows]            (m, row sum l)
+  //   part_o  [slots][n_parts][D / 8][part_rows][8]  unnormalised o
+  //   part_ml [slots][n_parts][part_rows]            (m, row sum l)
   // A tile of one part writes bf16 output directly.
   int32_t part_sub;
   int32_t n_parts;
+  int32_t part_rows;  // MFMA rows of the fullest tile
   float* part_o;
   float2* part_ml;
 };
 
-constexpr int kPrefillRows = 128;  // MFMA rows of a prefill query tile
 constexpr int kPrefillFewSub = 4;  // sub-tiles of a few-row tile's part: the LDS ring
 
 // The parts of a tile whose KV range holds kv positions: n of them, per
@@ -148,10 +148,13 @@ hipError_t rmsnorm(const void* x, int64_t x_stride, const void* residual, int64_
                    int64_t out_stride, int64_t rows, int hidden, float eps, hipStream_t stream);
 bool rmsnorm_supported(int hidden);
 
+// v_out not null (the append form): k_out / v_out are the [num_slots][hkv][D]
+// caches, written at out_loc[t].
 hipError_t qk_norm_rope(const void* qkv, int64_t stride, int64_t tokens, int hq, int hkv, int D,
                         const void* qw, const void* kw, const float* cos_t, const float* sin_t,
                         int64_t table_rows, const int32_t* positions, void* q_out, void* k_out,
-                        float eps, hipStream_t stream);
+                        float eps, void* v_out, int64_t num_slots, const int32_t* out_loc,
+                        hipStream_t stream);
 
 hipError_t silu_mul(const void* x, int64_t x_stride, int64_t rows, int inter, void* out,
                     int64_t out_stride, hipStream_t stream);
@@ -296,9 +299,8 @@ hipError_t launch_decode_combine(int D, const DecodeArgs& a, hipStream_t stream)
 
 hipError_t launch_prefill(int D, int NW, const PrefillArgs& a, int q_tiles, int batch,
                           hipStream_t stream);
-// The same with each tile's KV range split (a.part_sub > 0): rows_max = MFMA
-// rows of the fullest tile.
-hipError_t launch_prefill_split(int D, const PrefillArgs& a, int rows_max, hipStream_t stream);
+// The same with each tile's KV range split (a.part_sub > 0).
+hipError_t launch_prefill_split(int D, const PrefillArgs& a, hipStream_t stream);
 
 bool head_dim_supported(int D);
 bool group_supported(int G);

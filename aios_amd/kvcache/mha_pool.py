@@ -59,6 +59,11 @@ class MHAKVCache(BaseKVCache):
         )
 
     @property
+    def row_shape(self) -> tuple[int, int]:
+        """(num_kv_heads, head_dim) of a page's K or V row."""
+        return self._storage_shape[1:]
+
+    @property
     def device(self) -> torch.device:
         return self._device
 

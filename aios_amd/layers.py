@@ -15,7 +15,7 @@ from aios_amd import _lib
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _lib.raw_stream(t.device)
 
 
 def _check_rows(t: torch.Tensor, name: str) -> None:
@@ -70,6 +70,9 @@ class HipOps:
     # the attention backend, which applies the q/k RMSNorm + RoPE of
     # qk_norm_rope inside the decode launch.
     rope_in_decode = True
+    # ... and a prefill's K/V rows may be written to their pages by the launch
+    # that normalises and rotates them (qk_norm_rope_append).
+    rope_in_append = True
 
     @staticmethod
     def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -158,11 +161,7 @@ class HipOps:
                      num_qo_heads: int, num_kv_heads: int, head_dim: int,
                      eps: float) -> tuple[torch.Tensor, torch.Tensor]:
         """q, k = RoPE(RMSNorm_head(q)), RoPE(RMSNorm_head(k)) from qkv rows."""
-        _check_rows(qkv, "qkv")
-        if positions.dtype != torch.int32 or positions.numel() != qkv.shape[0]:
-            raise ValueError("positions must be int32 with one entry per token")
-        if cos.dtype != torch.float32 or cos.shape != sin.shape or cos.shape[1] != head_dim:
-            raise ValueError("cos/sin tables must be float32 [positions, head_dim]")
+        HipOps._check_rope(qkv, cos, sin, positions, head_dim)
         t = qkv.shape[0]
         q = torch.empty(t, num_qo_heads, head_dim, dtype=qkv.dtype, device=qkv.device)
         k = torch.empty(t, num_kv_heads, head_dim, dtype=qkv.dtype, device=qkv.device)
@@ -172,6 +171,42 @@ class HipOps:
             positions.contiguous().data_ptr(), q.data_ptr(), k.data_ptr(), eps, _stream(qkv)),
             "aios_qk_norm_rope")
         return q, k
+
+    @staticmethod
+    def _check_rope(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                    positions: torch.Tensor, head_dim: int) -> None:
+        _check_rows(qkv, "qkv")
+        if positions.dtype != torch.int32 or positions.numel() != qkv.shape[0]:
+            raise ValueError("positions must be int32 with one entry per token")
+        if cos.dtype != torch.float32 or cos.shape != sin.shape or cos.shape[1] != head_dim:
+            raise ValueError("cos/sin tables must be float32 [positions, head_dim]")
+
+    @staticmethod
+    def qk_norm_rope_append(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.Tensor,
+                            cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor,
+                            num_qo_heads: int, eps: float, k_cache: torch.Tensor,
+                            v_cache: torch.Tensor, out_loc: torch.Tensor) -> torch.Tensor:
+        """qk_norm_rope with the rotated K rows and qkv's V rows written to
+        rows out_loc of the contiguous bfloat16 [slots, Hkv, D] caches instead
+        of returned (store_kv in the same launch); returns q."""
+        _, num_kv_heads, head_dim = k_cache.shape
+        HipOps._check_rope(qkv, cos, sin, positions, head_dim)
+        t = qkv.shape[0]
+        if qkv.shape[1] != (num_qo_heads + 2 * num_kv_heads) * head_dim:
+            raise ValueError("qkv rows must hold the q, k and v heads")
+        for c in (k_cache, v_cache):
+            if c.dtype != torch.bfloat16 or c.shape != k_cache.shape or not c.is_contiguous():
+                raise ValueError("KV caches must be contiguous bfloat16 tensors of one shape")
+        if out_loc.dtype != torch.int32 or out_loc.numel() != t or not out_loc.is_contiguous():
+            raise ValueError("out_loc must be contiguous int32 with one entry per token")
+        q = torch.empty(t, num_qo_heads, head_dim, dtype=qkv.dtype, device=qkv.device)
+        _lib.check(_lib.lib().aios_qk_norm_rope_append(
+            qkv.data_ptr(), qkv.stride(0), t, num_qo_heads, num_kv_heads, head_dim,
+            q_weight.data_ptr(), k_weight.data_ptr(), cos.data_ptr(), sin.data_ptr(), cos.shape[0],
+            positions.contiguous().data_ptr(), q.data_ptr(), k_cache.data_ptr(),
+            v_cache.data_ptr(), k_cache.shape[0], out_loc.data_ptr(), eps, _stream(qkv)),
+            "aios_qk_norm_rope_append")
+        return q
 
     @staticmethod
     def attnres_mix(bank: torch.Tensor, partial: torch.Tensor | None,

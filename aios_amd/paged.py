@@ -14,7 +14,7 @@ DEFAULT_WORKSPACE = 128 * 1024 * 1024
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return _lib.raw_stream(device)
 
 
 def _host_i32(x) -> torch.Tensor:

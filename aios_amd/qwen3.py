@@ -128,7 +128,8 @@ class Qwen3ForCausalLM:
         """The attention of layer i between the qkv projection and o_proj:
         q/k norm + RoPE and the backend call -> [T, Hq, D] (or [T, Hq*D]).
         An appending decode batch on the gfx950 ops takes the norm and
-        rotation inside the decode launch (forward_rope)."""
+        rotation inside the decode launch (forward_rope); a prefill batch
+        writes K/V to their pages in the launch that rotates them."""
         c = self.config
         lw = self.w["layers"][i]
         t = qkv.shape[0]
@@ -143,6 +144,14 @@ class Qwen3ForCausalLM:
             out = be.forward_rope(q, k, v, lw["q_norm"], lw["k_norm"], self.rotary.cos_bf16,
                                   self.rotary.sin_bf16, positions, c.rms_norm_eps, kv_cache, i,
                                   batch)
+        elif (getattr(self.ops, "rope_in_append", False)
+                and getattr(be, "append_rope_applies", None) is not None
+                and be.append_rope_applies(qkv, kv_cache, batch)):
+            k_cache, v_cache = be.layer_kv(kv_cache, i)
+            q = self.ops.qk_norm_rope_append(qkv, lw["q_norm"], lw["k_norm"], self.rotary.cos,
+                                             self.rotary.sin, positions, hq, c.rms_norm_eps,
+                                             k_cache, v_cache, batch.out_loc.view(-1))
+            out = be.prefill_appended(q, k_cache, v_cache, batch)
         else:
             q, k = self.ops.qk_norm_rope(qkv, lw["q_norm"], lw["k_norm"], self.rotary.cos,
                                          self.rotary.sin, positions, hq, hkv, d, c.rms_norm_eps)

@@ -29,7 +29,7 @@ _NO_STEP_LIMIT = 2**31 - 1
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _lib.raw_stream(t.device)
 
 
 def stateless_uniforms(candidate_seeds: Sequence[int] | torch.Tensor, steps: int,

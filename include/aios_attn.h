@@ -331,6 +331,19 @@ int aios_qk_norm_rope(const void* qkv, int64_t qkv_stride, int64_t tokens, int32
                       float eps, void* stream);
 
 /*
+ * aios_qk_norm_rope followed by aios_kv_append of the rotated K rows and the V
+ * rows of qkv, in one launch: token t's rows go to k_cache[out_loc[t]] and
+ * v_cache[out_loc[t]] ([num_slots][Hkv][D] contiguous bf16 each; out_loc
+ * outside [0, num_slots) is skipped).  The same bits as the two calls.
+ */
+int aios_qk_norm_rope_append(const void* qkv, int64_t qkv_stride, int64_t tokens,
+                             int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,
+                             const void* q_weight, const void* k_weight, const float* cos_table,
+                             const float* sin_table, int64_t table_rows, const int32_t* positions,
+                             void* q_out, void* k_cache, void* v_cache, int64_t num_slots,
+                             const int32_t* out_loc, float eps, void* stream);
+
+/*
  * out[r][i] = bf16(bf16(silu(x[r][i])) * x[r][intermediate + i]) for the
  * merged gate/up rows x [rows][2 * intermediate].  Replaces silu_and_mul
  * (python/aios/layers/activation.py:9-12).

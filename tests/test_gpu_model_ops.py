@@ -65,6 +65,29 @@ def test_qk_norm_rope(hq, hkv, d):
     _ulp_close(q1[:1], xn)
 
 
+@pytest.mark.parametrize("hq,hkv,d,t", [(8, 2, 96, 1), (12, 4, 64, 19), (16, 8, 128, 5),
+                                        (8, 8, 64, 3), (32, 8, 128, 130)])
+def test_qk_norm_rope_append_is_the_two_calls(hq, hkv, d, t):
+    """The same bits as qk_norm_rope and store_cache, rows of other slots left
+    alone, slots outside the pool skipped; qkv rows with a gap between them."""
+    from aios_amd.kernel import store_cache
+
+    qkv = _bf16((t, (hq + 2 * hkv) * d + 6), d + hq, 1.5)[:, : (hq + 2 * hkv) * d]
+    qw, kw = _bf16((d,), 3).abs() + 0.5, _bf16((d,), 4).abs() + 0.5
+    rot = RotaryEmbedding(d, 512, 1000000.0, DEV)
+    pos = (torch.arange(t, device=DEV, dtype=torch.int32) * 37) % 600  # some past the table
+    loc = torch.randperm(t + 9, generator=torch.Generator().manual_seed(t))[:t].to(torch.int32)
+    if t > 2:
+        loc[1], loc[2] = -1, t + 9
+    loc = loc.to(DEV)
+    kc, vc = _bf16((t + 9, hkv, d), 5), _bf16((t + 9, hkv, d), 6)
+    k2, v2 = kc.clone(), vc.clone()
+    q1, k1 = HipOps.qk_norm_rope(qkv, qw, kw, rot.cos, rot.sin, pos, hq, hkv, d, 1e-6)
+    store_cache(kc, vc, loc, k1, qkv[:, (hq + hkv) * d:].view(t, hkv, d))
+    q2 = HipOps.qk_norm_rope_append(qkv, qw, kw, rot.cos, rot.sin, pos, hq, 1e-6, k2, v2, loc)
+    assert torch.equal(q1, q2) and torch.equal(kc, k2) and torch.equal(vc, v2)
+
+
 @pytest.mark.parametrize("rows,inter", [(8, 2048), (32, 3072), (3, 9728)])
 def test_silu_and_mul(rows, inter):
     x = _bf16((rows, 2 * inter), inter, 2.0)
