@@ -79,7 +79,10 @@ template <int MT, int PRO, int EPI, int KS = 0, int NC = 16>
 __global__ __launch_bounds__(kGemmThreads) void skinny_gemm_kernel(AIOS_LINEAR_HOT_PARAMS) {
   AIOS_LINEAR_HOT_BIND
   static_assert(NC == 16 || ((NC == 8 || NC == 4) && MT == 1), "narrow tiles: one row tile");
-  constexpr int NP = EPI == kSiluPair ? 2 : 1;  // W row sets per workgroup
+  // SiLU with 8 columns: the 8 gate rows and the 8 up rows are one MFMA tile
+  // (half the loads and MFMAs of two half-empty ones).
+  constexpr bool MERGED = EPI == kSiluPair && NC == 8;
+  constexpr int NP = EPI == kSiluPair && !MERGED ? 2 : 1;  // W row sets per workgroup
   __shared__ f32x4 red[3][NP][MT][64];
   __shared__ float ssq[4][MT][16];
   const int lane = threadIdx.x & 63;
@@ -90,9 +93,9 @@ __global__ __launch_bounds__(kGemmThreads) void skinny_gemm_kernel(AIOS_LINEAR_H
   const int kq = a.K >> 2;  // multiple of 32
   const int k_begin = wave * kq + lg * 8;
   const int steps = KS > 0 ? KS : kq >> 5;
-  const bool wok = NC == 16 || l16 < NC;  // this lane's W row is one of the tile's
+  const bool wok = NC == 16 || MERGED || l16 < NC;  // this lane's W row is one of the tile's
   const bf16* wrow[NP];
-  wrow[0] = a.w + (n0 + (wok ? l16 : 0)) * a.w_stride + k_begin;
+  wrow[0] = a.w + (n0 + (MERGED && l16 >= 8 ? a.N + l16 - 8 : wok ? l16 : 0)) * a.w_stride + k_begin;
   if constexpr (NP == 2) wrow[NP - 1] = a.w + (a.N + n0 + (wok ? l16 : 0)) * a.w_stride + k_begin;
   int64_t xoff[MT], roff[MT];
   bool xok[MT];
@@ -252,9 +255,17 @@ __global__ __launch_bounds__(kGemmThreads) void skinny_gemm_kernel(AIOS_LINEAR_H
 #pragma unroll
     for (int p = 0; p < NP; ++p)
       v[p] = acc[p][mt] + red[0][p][mt][lane] + red[1][p][mt][lane] + red[2][p][mt][lane];
+    if constexpr (MERGED) {  // lanes lg 0, 1: gate columns; the up columns 32 lanes on
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float up = round_bf16(__shfl_xor(v[0][i], 32));
+        const float g = round_bf16(v[0][i]);
+        v[0][i] = round_bf16(g / (1.f + expf(-g))) * up;
+      }
+    }
     if (!xok[mt]) continue;
     f32x4 o = v[0];
-    if constexpr (EPI == kSiluPair) {
+    if constexpr (NP == 2) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float g = round_bf16(v[0][i]);
