@@ -780,8 +780,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
 //     or below the bound are an upper set of the sampling logits with at
 //     least k members, so they hold the top k;
 //  4. those candidates are written to LDS as composite keys (value key above
-//     ~id: distinct, larger = higher value, then lower id) at positions from
-//     per-slot ballots, and ordered: up to kResRankMax of them by rank
+//     ~id: distinct, larger = higher value, then lower id), in no order, and
+//     ordered: up to kResRankMax of them by rank
 //     counting (several threads per candidate, each over a contiguous run),
 //     more by a bitonic sort;
 //  5. more than kResCap candidates (ids tied at the bound): the k-th value
@@ -795,7 +795,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
 // ids and 9.6 us at 6400, against 40-48 us for sample_kernel's three sweeps.
 constexpr int kResMaxVocab = 16384;  // ids per row at most
 constexpr int kResCap = 2048;     // candidates gathered and ordered at most
-constexpr int kResRankMax = 256;  // candidates ordered by rank counting at most
+constexpr int kResRankMax = 1024;  // candidates ordered by rank counting at most
 static_assert(kResCap >= kSampleMaxTopK, "the exact top k fits the candidate buffer");
 
 template <typename T>
@@ -818,7 +818,7 @@ struct ResSelect {
   alignas(16) uint32_t red[2][NW][8];  // per-wavefront packed counts
   float fred[2][NW][2];                // per-wavefront max / sum
   uint32_t ired[2][NW];                // per-wavefront counts (bisection)
-  uint32_t gscan[NW];                  // per-wavefront candidate counts
+  uint32_t taken;                      // candidates gathered
 };
 template <typename Key>
 struct ResOrder {
@@ -1025,6 +1025,7 @@ __device__ __forceinline__ ResSelected res_select(const SampleArgs& a, ResSelect
   }
   // 1. forbidden bitmap
   for (int i = tid; i < (vocab + 31) / 32; i += NT) sh.fbits[i] = 0u;
+  if (tid == 0) sh.taken = 0u;
   __syncthreads();
   if (fid >= 0) atomicOr(&sh.fbits[fid >> 5], 1u << (fid & 31));
 
@@ -1123,38 +1124,20 @@ __device__ __forceinline__ ResSelected res_select(const SampleArgs& a, ResSelect
   auto ckey = [&](int c, int j) {
     return ((Key)res_vkey(v[c][j], (T*)nullptr) << kIdBits) | (kIdMask - (Key)(id0 + id_of(c, j)));
   };
-  // Writes the ids for which pred(c, j) holds to cand (wavefront by
-  // wavefront, id slot by id slot: one ballot per slot, positions from the
-  // wavefront totals and mbcnt); returns how many.
+  // Writes the ids for which pred(c, j) holds to cand, in no order; returns
+  // how many.  (Called once; few ids of a wavefront hold, so an LDS counter
+  // costs less than a ballot per id slot.)
   auto gather = [&](auto&& pred) -> int {
-    uint32_t wcnt = 0u;
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) wcnt += __popcll(__ballot(pred(c, j)));
-    if (lane == 0) sh.gscan[wave] = wcnt;
-    __syncthreads();
-    uint32_t pos = 0u, total = 0u;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const uint32_t t = sh.gscan[w];
-      pos += w < wave ? t : 0u;
-      total += t;
-    }
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const bool pr = pred(c, j);
-        const uint64_t mk = __ballot(pr);
-        if (mk != 0ull) {
-          const uint32_t at = pos + __builtin_amdgcn_mbcnt_hi(
-                                        (uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0u));
-          if (pr && at < (uint32_t)kResCap) cand[at] = ckey(c, j);
-          pos += __popcll(mk);
+      for (int j = 0; j < 8; ++j)
+        if (pred(c, j)) {
+          const uint32_t at = atomicAdd(&sh.taken, 1u);
+          if (at < (uint32_t)kResCap) cand[at] = ckey(c, j);
         }
-      }
-    return (int)min(total, (uint32_t)kResCap);
+    __syncthreads();
+    return (int)min(sh.taken, (uint32_t)kResCap);
   };
 
   auto in_row = [&](int c, int j) { return ((valid >> (8 * c + j)) & 1u) != 0u; };
@@ -1237,34 +1220,46 @@ __device__ __forceinline__ void res_pick(const SampleArgs& a, ResOrder<Key>& sh,
   while (npad < n) npad <<= 1;
   for (int i = n + tid; i < npad; i += NT) sh.cand[i] = 0;
   __syncthreads();
-  if (n <= kResRankMax) {
+  constexpr int KV = 16 / sizeof(Key);  // keys per 16-byte read
+  // How many of the len entries from run on are larger than ce.
+  auto larger = [&](const Key* run, int len, Key ce) {
+    int r = 0;
+    if (len % KV == 0) {
+      for (int j = 0; j < len; j += KV) {
+        const uint4 q = *reinterpret_cast<const uint4*>(run + j);
+        if constexpr (KV == 4) {
+          r += (q.x > ce ? 1 : 0) + (q.y > ce ? 1 : 0) + (q.z > ce ? 1 : 0) + (q.w > ce ? 1 : 0);
+        } else {
+          r += ((((Key)q.y << 32) | q.x) > ce ? 1 : 0) + ((((Key)q.w << 32) | q.z) > ce ? 1 : 0);
+        }
+      }
+    } else {
+      for (int j = 0; j < len; ++j) r += run[j] > ce ? 1 : 0;
+    }
+    return r;
+  };
+  if (npad <= NT) {
     // tpe threads per candidate, each counting the larger keys in its own
     // contiguous run of L entries
     const int tpe = min(min(64, NT / npad), npad);
-    const int L = npad / tpe;
+    const int L = tpe == 1 && npad >= KV ? (n + KV - 1) / KV * KV : npad / tpe;
     const int e = tid / tpe;
     const int p = tid - e * tpe;
     int r = 0;
     Key ce = 0;
     if (e < n) {
       ce = sh.cand[e];
-      const Key* run = sh.cand + p * L;
-      constexpr int KV = 16 / sizeof(Key);  // keys per 16-byte read
-      if (L % KV == 0) {
-        for (int j = 0; j < L; j += KV) {
-          const uint4 q = *reinterpret_cast<const uint4*>(run + j);
-          if constexpr (KV == 4) {
-            r += (q.x > ce ? 1 : 0) + (q.y > ce ? 1 : 0) + (q.z > ce ? 1 : 0) + (q.w > ce ? 1 : 0);
-          } else {
-            r += ((((Key)q.y << 32) | q.x) > ce ? 1 : 0) + ((((Key)q.w << 32) | q.z) > ce ? 1 : 0);
-          }
-        }
-      } else {
-        for (int j = 0; j < L; ++j) r += run[j] > ce ? 1 : 0;
-      }
+      r = larger(sh.cand + p * L, L, ce);
     }
     for (int off = 1; off < tpe; off <<= 1) r += __shfl_xor(r, off);
     if (e < n && p == 0 && r < k) sh.top[r] = ce;
+    __syncthreads();
+  } else if (n <= kResRankMax) {
+    for (int e = tid; e < n; e += NT) {
+      const Key ce = sh.cand[e];
+      const int r = larger(sh.cand, (n + KV - 1) / KV * KV, ce);
+      if (r < k) sh.top[r] = ce;
+    }
     __syncthreads();
   } else {
     for (int size = 2; size <= npad; size <<= 1) {
