@@ -9,6 +9,8 @@ import ctypes
 import threading
 from pathlib import Path
 
+import torch
+
 LIB_PATH = Path(__file__).resolve().parent / "libaios_attn.so"
 
 AIOS_OK = 0
@@ -103,8 +105,6 @@ class AttnPlan(ctypes.Structure):
 def raw_stream(device) -> int:
     """The current HIP stream handle of a torch GPU device (the handle alone:
     torch.cuda.current_stream builds a Stream object, 2 us of each launch)."""
-    import torch
-
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 

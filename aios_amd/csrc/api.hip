@@ -253,6 +253,35 @@ int aios_attn_plan(int32_t phase, const int32_t* cu_q, const int32_t* cu_k, int3
     split = pass;
   }
   int32_t n_splits = max_suffix > 0 ? cdiv(max_suffix, split) : 1;
+  // One prefix workgroup per compute unit makes short chunks of a short
+  // prefix.  Up to the four sub-tiles that a workgroup requests at once a
+  // longer chunk may cost less: a sub-tile adds about 300 ns, every workgroup
+  // (prefix and suffix) past one per unit 4.5 ns (two on a unit slow each
+  // other down), past two per unit, the most that are resident, 20 ns more,
+  // and every part 30 ns of the combine.  Fitted to chunks of 32 to
+  // 128 over 13 shapes (main + combine per layer): 16 rows of 12q/4kv x 64 over
+  // 4,000 positions 64 / 96 / 128: 9.0 / 8.2 / 8.2 us; 40 rows of 32q/8kv x 128
+  // over 1,000: 11.7 / 9.4 / 9.6; 24 rows over 400, 32 / 64 / 96: 8.2 / 7.9 /
+  // 8.4.  With at most 32 query rows one wavefront computes and sharing a unit
+  // costs nothing (8 rows of 16q/8kv x 128 over 2,000: 8.3 / 8.7 / 8.6): kept.
+  if (cascade && prefix_chunk_len <= 0 && m_rows > 32) {
+    int64_t best = 0;
+    int32_t pick = chunk;
+    for (int32_t c = chunk; c <= 4 * 32; c += 32) {
+      const int64_t n = cdiv(P, c);
+      const int64_t wgs = hkv * (mgroups * n + (int64_t)batch * n_splits);
+      const int64_t ns = 300 * (c / 32) + (wgs > cus ? 9 * (wgs - cus) / 2 : 0) +
+                         (wgs > 2 * cus ? 20 * (wgs - 2 * cus) : 0) + 30 * n;
+      if (c == chunk) {
+        best = ns - 400;  // (a closer call is not a gain to rely on)
+      } else if (ns < best) {
+        best = ns;
+        pick = c;
+      }
+    }
+    chunk = pick;
+    n_chunks = cdiv(P, chunk);
+  }
   // Bound the parts per (row, kv-head) merged by the combine.
   while (n_chunks + n_splits > kMaxParts) {
     if (n_splits > n_chunks) {
@@ -446,8 +475,8 @@ int decode_impl(const aios_attn_plan_t* p, const void* q, int64_t q_tok_stride,
   a.chunk_len = p->prefix_chunk_len;
   a.n_chunks = p->num_prefix_chunks;
   a.m_rows = p->cascade_rows;
-  a.m_groups = p->cascade_mgroups > 0 ? p->cascade_mgroups : 1;
-  a.prefix_wgs = p->num_prefix_chunks * p->num_kv_heads * a.m_groups;
+  a.prefix_units = p->num_prefix_chunks * p->num_kv_heads;
+  a.prefix_wgs = a.prefix_units * (p->cascade_mgroups > 0 ? p->cascade_mgroups : 1);
   a.split_len = p->suffix_split_len;
   a.n_splits = p->num_suffix_splits;
   a.suffix_items = p->batch_size * p->num_kv_heads * p->num_suffix_splits;

@@ -47,8 +47,13 @@ __device__ __forceinline__ void decode_prefix_part(uint8_t* lds, const DecodeArg
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int hl = lane >> 5;
-  const int mg = wg % a.m_groups;
-  const int unit = wg / a.m_groups;
+  // The row groups of a chunk (more than 128 query rows) are a whole pass over
+  // the (chunk, kv-head) units apart, so that with 8 kv-heads they run on one
+  // XCD, at about the same time, and share its L2's copy of the chunk
+  // (64 rows of 32q/8kv x 128 over 4,000 positions: 20.2 -> 16.1 us per layer
+  // against neighbouring workgroups, on two XCDs).
+  const int mg = wg / a.prefix_units;
+  const int unit = wg % a.prefix_units;
   // Consecutive workgroups take different kv-heads: the hardware deals
   // workgroups round-robin to the XCDs, so with 8 kv-heads every chunk of
   // one head (and the combine of that head, which uses the same order) runs
@@ -584,20 +589,20 @@ struct DecodeHot {
   const int32_t* indices;
   const int32_t* cu_k;
   const int32_t* out_loc;  // null: no fused append
-  int32_t prefix_wgs, prefix_len, chunk_len, m_groups, num_kv_heads, splits_flags, split_len,
+  int32_t prefix_wgs, prefix_len, chunk_len, prefix_units, num_kv_heads, splits_flags, split_len,
       m_rows;
 };
 __host__ __device__ inline DecodeHot decode_hot(const DecodeArgs& a) {
   const int32_t sf = a.n_splits | (a.final_out ? 1 << 16 : 0) | (a.wave_parts ? 1 << 17 : 0);
   return DecodeHot{a.indices,  a.cu_k,         a.out_loc, a.prefix_wgs, a.prefix_len, a.chunk_len,
-                   a.m_groups, a.num_kv_heads, sf,        a.split_len,  a.m_rows};
+                   a.prefix_units, a.num_kv_heads, sf,        a.split_len,  a.m_rows};
 }
 
 template <int D, int G, bool ROPE>
 __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_main_kernel(
     const int32_t* __restrict__ indices, const int32_t* __restrict__ cu_k,
     const int32_t* __restrict__ out_loc, int32_t prefix_wgs,
-    int32_t prefix_len, int32_t chunk_len, int32_t m_groups, int32_t num_kv_heads,
+    int32_t prefix_len, int32_t chunk_len, int32_t prefix_units, int32_t num_kv_heads,
     int32_t splits_flags, int32_t split_len, int32_t m_rows, DecodeArgs args) {
   __shared__ __align__(16) uint8_t lds[decode_lds_bytes<D, G>()];
   DecodeArgs a = args;
@@ -607,7 +612,7 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
   a.prefix_wgs = prefix_wgs;
   a.prefix_len = prefix_len;
   a.chunk_len = chunk_len;
-  a.m_groups = m_groups;
+  a.prefix_units = prefix_units;
   a.num_kv_heads = num_kv_heads;
   a.n_splits = splits_flags & 0xffff;
   a.final_out = (splits_flags >> 16) & 1;
@@ -640,12 +645,12 @@ static hipError_t launch_main_dg(const DecodeArgs& a, hipStream_t s) {
   if (a.q_norm != nullptr)
     hipLaunchKernelGGL((decode_main_kernel<D, G, true>), grid, dim3(kEngineThreads), 0, s,
                        h.indices, h.cu_k, h.out_loc, h.prefix_wgs, h.prefix_len, h.chunk_len,
-                       h.m_groups,
+                       h.prefix_units,
                        h.num_kv_heads, h.splits_flags, h.split_len, h.m_rows, a);
   else
     hipLaunchKernelGGL((decode_main_kernel<D, G, false>), grid, dim3(kEngineThreads), 0, s,
                        h.indices, h.cu_k, h.out_loc, h.prefix_wgs, h.prefix_len, h.chunk_len,
-                       h.m_groups,
+                       h.prefix_units,
                        h.num_kv_heads, h.splits_flags, h.split_len, h.m_rows, a);
   return hipGetLastError();
 }

@@ -54,8 +54,8 @@ struct DecodeArgs {
   int32_t chunk_len;
   int32_t n_chunks;
   int32_t m_rows;      // batch * group
-  int32_t m_groups;
-  int32_t prefix_wgs;  // n_chunks * Hkv * m_groups
+  int32_t prefix_units;  // n_chunks * Hkv
+  int32_t prefix_wgs;    // prefix_units * groups of 128 query rows
   // per-row suffix work: (row, kv-head, split) items, one wavefront each
   int32_t split_len;
   int32_t n_splits;

@@ -90,6 +90,41 @@ def test_plan_decode_long_rows_without_prefix_split():
     assert p.suffix_parts_per_item == 1 and p.num_parts == p.num_suffix_splits
 
 
+@pytest.mark.parametrize("rows,prefix,hq,hkv,d,chunk", [
+    (12, 1000, 32, 8, 128, 64),    # 352 workgroups at 32: lengthened to fit the units
+    (8, 2000, 16, 8, 128, 64),     # one wavefront of rows: one workgroup per unit
+    (64, 2000, 16, 8, 128, 128),   # more than two per unit: the longest burst
+    (24, 4096, 32, 8, 128, 128),
+    (48, 16000, 16, 8, 128, 512),  # chunks past four sub-tiles: one workgroup per unit
+])
+def test_plan_decode_chunk_length(rows, prefix, hq, hkv, d, chunk):
+    kv = np.cumsum([0] + [prefix + 31] * rows)
+    rc, p = _plan(_lib.PHASE_DECODE, np.arange(rows + 1), kv, hq=hq, hkv=hkv, d=d, shared=prefix)
+    assert rc == 0 and p.prefix_chunk_len == chunk
+    assert (p.num_prefix_chunks - 1) * chunk < prefix <= p.num_prefix_chunks * chunk
+    assert p.num_parts <= 64
+
+
+@pytest.mark.parametrize("q,kv,hq,hkv,d", [(6, 4099, 32, 8, 128), (1, 193, 8, 8, 64),
+                                          (100, 4100, 32, 8, 128), (2048, 2048, 16, 8, 128),
+                                          (4096, 4096, 32, 8, 128), (8, 150, 32, 8, 128)])
+def test_plan_prefill_split(q, kv, hq, hkv, d):
+    """The parts of the longest tile cover its range, the workspace holds every
+    part's state, and a workspace limit below it leaves the batch unsplit."""
+    rc, p = _plan(_lib.PHASE_PREFILL, [0, q], [0, kv], hq=hq, hkv=hkv, d=d, ws=1 << 27)
+    assert rc == 0
+    if p.num_parts == 0:
+        assert p.ws_bytes == 0 and (q, kv) in ((4096, 4096), (8, 150))
+        return
+    assert p.num_parts > 1 and p.prefix_chunk_len % 32 == 0
+    assert p.num_parts * p.prefix_chunk_len >= kv
+    states = p.num_q_tiles * hkv * p.num_parts * min(q, p.prefill_q_tile) * p.group
+    assert p.ws_parts_lse >= states * d * 4 and p.ws_bytes >= p.ws_parts_lse + states * 8
+    rc, small = _plan(_lib.PHASE_PREFILL, [0, q], [0, kv], hq=hq, hkv=hkv, d=d,
+                      ws=p.ws_bytes - 1)
+    assert rc == 0 and small.num_parts == 0 and small.ws_bytes == 0
+
+
 def test_plan_rejects_bad_batches():
     lib = _lib.lib()
     rc, _ = _plan(_lib.PHASE_DECODE, [0, 2], [0, 5])  # two query tokens in decode
