@@ -79,6 +79,22 @@ def test_attnres_mix_matches_oracle(s, n, d, with_partial):
     assert bool((scores[total:] == 123.0).all())  # rows past the sources untouched
 
 
+@pytest.mark.parametrize("with_partial", [False, True])
+@pytest.mark.parametrize("total", range(2, 18))
+def test_attnres_every_source_count(total, with_partial):
+    """Each built source count of the one-wavefront kernel and the first past
+    it, at the three hidden sizes; scores to fp32 rounding of 1024-term sums."""
+    s = total - int(with_partial)
+    for n, d in ((3, 512), (5, 768), (2, 1024)):
+        bank, partial, query, knw, wq = _inputs(s, n, d, with_partial, 500 + total + d)
+        scores = torch.full((total + 1, n), 123.0, device=DEV)
+        out = attnres_mix(bank, partial, wq, 1e-6, score_buffer=scores)
+        _check(out, oar.mix(_np(bank), _np(partial), _np(query), _np(knw), 1e-6))
+        want = oar.scores(_np(bank), _np(partial), _np(query), _np(knw), 1e-6)
+        assert np.allclose(scores[:total].cpu().numpy(), want, rtol=1e-4, atol=1e-4)
+        assert bool((scores[total:] == 123.0).all())
+
+
 def test_attnres_zero_query_is_uniform_mean():
     """tests/test_ime_attnres.py:59-66 on the GPU (values exact in bf16)."""
     bank = torch.arange(3 * 2 * 8, dtype=torch.float32, device=DEV).reshape(3, 2, 8)
