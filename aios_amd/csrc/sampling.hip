@@ -1125,16 +1125,29 @@ __device__ __forceinline__ ResSelected res_select(const SampleArgs& a, ResSelect
     return ((Key)res_vkey(v[c][j], (T*)nullptr) << kIdBits) | (kIdMask - (Key)(id0 + id_of(c, j)));
   };
   // Writes the ids for which pred(c, j) holds to cand, in no order; returns
-  // how many.  (Called once; few ids of a wavefront hold, so an LDS counter
-  // costs less than a ballot per id slot.)
+  // how many.  (Called once.  One scan of the lanes' counts and one step of an
+  // LDS counter per wavefront: with a counter step per id the wavefront waits
+  // for a round trip each, 24 rows of 16,384 ids, top_k 96 / 160: 14.9 / 17.6
+  // us, now 13.7 / 15.7.)
+  static_assert(NC <= 4, "a thread's ids fit a 32-bit mask");
   auto gather = [&](auto&& pred) -> int {
+    uint32_t hits = 0u;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) hits |= pred(c, j) ? 1u << (8 * c + j) : 0u;
+    const uint32_t mine = (uint32_t)__popc(hits);
+    const uint32_t ends = lanes_scan_u(mine);
+    uint32_t at = 0u;
+    if (lane == 63 && ends != 0u) at = atomicAdd(&sh.taken, ends);
+    at = (uint32_t)__builtin_amdgcn_readlane((int)at, 63) + ends - mine;
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        if (pred(c, j)) {
-          const uint32_t at = atomicAdd(&sh.taken, 1u);
+        if (hits & (1u << (8 * c + j))) {
           if (at < (uint32_t)kResCap) cand[at] = ckey(c, j);
+          ++at;
         }
     __syncthreads();
     return (int)min(sh.taken, (uint32_t)kResCap);
@@ -1365,7 +1378,7 @@ __global__ __launch_bounds__(NT) void sample_resident_kernel(SampleArgs a) {
 // which is ordered and sampled as there.  One workgroup per row alone took
 // 376 us for 24 bf16 rows of 151,936 ids, top_k 50 (sample_kernel: three sweeps
 // of one compute unit with up to 16 compares per id);
-// split, 12.1 us for the segments and 6.8 us for the merge.
+// split, 18.4 us for both launches.
 constexpr int kSegThreads = 512;
 constexpr int kSegIds = 8192;
 constexpr int kMaxSegs = 64;          // segments of a row (one lane each in the merge)
