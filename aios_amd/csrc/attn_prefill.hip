@@ -84,7 +84,7 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
 // traffic.  Measured per layer on MI355X (graph replay), one workgroup per
 // tile -> split (main launch + combine): 6 tokens against 4,099 positions,
 // 32q/8kv x 128: 94.7 -> 16.2 us; 100 against 4,100: 102 -> 28 us; a
-// 2,048-token prompt, 16q/8kv x 128: 58 -> 47 us.
+// 2,048-token prompt, 16q/8kv x 128: 57 -> 42 us.
 //
 // A tile of at most 64 rows fills one or two of the four 32-row wavefront
 // tiles; its wavefronts then also share the part's sub-tiles (all resident
