@@ -131,7 +131,8 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
   const int kv_end = min(kv_hi, kv_begin + pp.per * kSubTok);
 
   // Wavefront -> (row tile, share of the sub-tiles).
-  const int rows = (q_hi - qt * a.q_tile) * G;
+  // (at most what the plan gave each part room for)
+  const int rows = min((q_hi - qt * a.q_tile) * G, a.part_rows);
   const int nr = rows <= 32 ? 1 : rows <= 64 ? 2 : 4;
   const int rt = wave & (nr - 1);
   const int share = nr == 4 ? 0 : nr == 2 ? wave >> 1 : wave;
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_combine_kernel(PrefillArgs a,
   const int q_hi = min(q_len, (qt + 1) * a.q_tile);
   const PrefillParts pp =
       prefill_parts(min(kv_len, kv_len - q_len + q_hi), a.part_sub, a.n_parts);
-  const int rows = (q_hi - qt * a.q_tile) * a.group;
+  const int rows = min((q_hi - qt * a.q_tile) * a.group, a.part_rows);
   if (pp.n == 1 || rb * RB >= rows) return;  // (uniform)
   const int dg = lane % DG;
   const int m = rb * RB + lane / DG;
