@@ -104,7 +104,10 @@ class AttnPlan(ctypes.Structure):
 
 def raw_stream(device) -> int:
     """The current HIP stream handle of a torch GPU device (the handle alone:
-    torch.cuda.current_stream builds a Stream object, 2 us of each launch)."""
+    torch.cuda.current_stream builds a Stream object, 2 us of each launch).
+    Another device has none: its tensors' addresses must not reach a kernel."""
+    if device.type != "cuda":
+        raise ValueError(f"expected a GPU device, got {device}")
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 

@@ -18,6 +18,12 @@ def _stream(t: torch.Tensor) -> int:
     return _lib.raw_stream(t.device)
 
 
+def _check_gpu(*tensors: torch.Tensor) -> None:
+    for t in tensors:
+        if not t.is_cuda:
+            raise ValueError("the kernels take GPU tensors")
+
+
 def _check_rows(t: torch.Tensor, name: str) -> None:
     if t.dtype != torch.bfloat16 or not t.is_cuda or t.ndim != 2 or t.stride(1) != 1:
         raise ValueError(f"{name} must be a 2-D bfloat16 GPU tensor with contiguous rows")
@@ -48,6 +54,7 @@ def _add_rmsnorm(h: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
 
 def _linear_rows(x: torch.Tensor, weight: torch.Tensor, n: int, silu: bool = False) -> torch.Tensor:
     """The few-row projection (aios_linear_rows_ws) to n columns."""
+    _check_gpu(x, weight)
     rows, k = x.shape
     lib = _lib.lib()
     y = torch.empty(rows, n, dtype=x.dtype, device=x.device)
@@ -111,6 +118,7 @@ class HipOps:
         if (rows_ok and rows <= 16 and k <= 1024
                 and (residual is None
                      or (residual.stride(1) == 1 and residual.stride(0) % 8 == 0))):
+            _check_gpu(h, weight, norm_weight, *(() if residual is None else (residual,)))
             y = torch.empty(rows, n, dtype=h.dtype, device=h.device)
             total = torch.empty_like(h) if residual is not None else h
             _lib.check(_lib.lib().aios_linear_rows_ex(
@@ -197,6 +205,7 @@ class HipOps:
         for c in (k_cache, v_cache):
             if c.dtype != torch.bfloat16 or c.shape != k_cache.shape or not c.is_contiguous():
                 raise ValueError("KV caches must be contiguous bfloat16 tensors of one shape")
+        _check_gpu(k_cache, v_cache, out_loc)
         if out_loc.dtype != torch.int32 or out_loc.numel() != t or not out_loc.is_contiguous():
             raise ValueError("out_loc must be contiguous int32 with one entry per token")
         q = torch.empty(t, num_qo_heads, head_dim, dtype=qkv.dtype, device=qkv.device)

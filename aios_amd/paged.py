@@ -252,8 +252,8 @@ def prefill(p: _lib.AttnPlan, q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
 def build_indices(page_table: torch.Tensor, row_ids: torch.Tensor, cu_k: torch.Tensor,
                   total_kv: int) -> torch.Tensor:
     """Device gather of the flat page-index list (aios_build_indices)."""
-    if page_table.dtype != torch.int32 or page_table.stride(1) != 1:
-        raise ValueError("page_table must be int32 with contiguous rows")
+    if page_table.dtype != torch.int32 or page_table.stride(1) != 1 or not page_table.is_cuda:
+        raise ValueError("page_table must be an int32 GPU tensor with contiguous rows")
     _check_i32(row_ids, "row_ids", 0)
     _check_i32(cu_k, "cu_k", row_ids.numel() + 1)
     out = torch.empty(total_kv, dtype=torch.int32, device=page_table.device)
@@ -374,6 +374,8 @@ def bind_kv_append(k_cache: torch.Tensor, v_cache: torch.Tensor, out_loc: torch.
         raise ValueError("K/V input shape does not match the cache layout")
     if out_loc.dtype != torch.int32 or not out_loc.is_contiguous() or out_loc.numel() != k.shape[0]:
         raise ValueError("out_loc must be a contiguous int32 tensor with one entry per token")
+    if not all(t.is_cuda for t in (k_cache, v_cache, out_loc, k, v)):
+        raise ValueError("the KV append takes GPU tensors")
     s = stream.cuda_stream if stream is not None else _stream(k.device)
     width = k_cache.shape[1] * k_cache.shape[2]
     args = (k_cache.data_ptr(), v_cache.data_ptr(), k_cache.shape[0], k_cache.stride(0),

@@ -5,9 +5,11 @@ from __future__ import annotations
 import pytest
 import torch
 
+from aios_amd import _lib, paged
 from aios_amd.core import Req, SamplingParams
 from aios_amd.ime import (Candidate, CandidateGroupConfig, adaptive_refill_attempts,
                            candidate_valid, select_top, token_longest_common_prefix)
+from aios_amd.layers import HipOps
 from aios_amd.scheduler import CacheManager
 from oracle import prefix as oprefix
 
@@ -185,3 +187,89 @@ def test_refill_ban_fill_defaults_to_the_model_pad_id():
     assert config_from_hf(config_to_hf(c)).pad_token_id == 7
     assert "pad_token_id" not in config_to_hf(MINIMIND_0P1B)
     assert config_from_hf(config_to_hf(MINIMIND_0P1B)).pad_token_id is None
+
+
+class _NoLaunch:
+    """Stands for the library: any entry point that is called is recorded."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def entry(*args):
+            self.calls.append(name)
+            return 0
+
+        return entry
+
+
+def _host_calls():
+    bf = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16)
+    i32 = lambda *shape: torch.zeros(shape, dtype=torch.int32)
+    ops = HipOps()
+    cache, kv = bf(4, 2, 64), bf(3, 2, 64)
+    append = lambda: ops.qk_norm_rope_append(bf(3, 8 * 64), bf(64), bf(64), torch.zeros(9, 64),
+                                             torch.zeros(9, 64), i32(3), 4, 1e-6, cache, cache,
+                                             i32(3))
+    return {
+        "linear": lambda: ops.linear(bf(3, 128), bf(16, 128)),
+        "add_rmsnorm_linear": lambda: ops.add_rmsnorm_linear(bf(3, 128), bf(3, 128), bf(128), 1e-6,
+                                                             bf(16, 128)),
+        "add_rmsnorm_linear_wide": lambda: ops.add_rmsnorm_linear(bf(3, 2560), bf(3, 2560),
+                                                                  bf(2560), 1e-6, bf(16, 2560)),
+        "qk_norm_rope_append": append,
+        "build_indices": lambda: paged.build_indices(i32(2, 8), i32(2), i32(3), 4),
+        "bind_kv_append": lambda: paged.bind_kv_append(cache, cache, i32(3), kv, kv)(),
+        "raw_stream": lambda: _lib.raw_stream(torch.device("cpu")),
+        "raw_stream_meta": lambda: _lib.raw_stream(torch.device("meta")),
+    }
+
+
+@pytest.mark.parametrize("name", sorted(_host_calls()))
+def test_host_tensors_never_reach_a_kernel(name, monkeypatch):
+    """A call on CPU tensors is refused before any launch, also where a GPU is
+    current (its stream and index stand in here)."""
+    lib = _NoLaunch()
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0, raising=False)
+    with pytest.raises(ValueError):
+        _host_calls()[name]()
+    assert lib.calls == []
+
+
+class _GpuTensor(torch.Tensor):
+    """A CPU tensor that says it is on the GPU (for a call's checks of its other operands)."""
+
+    is_cuda = True
+
+
+@pytest.mark.parametrize("on_host", ["page_table", "row_ids", "k_cache", "v_cache", "out_loc", "k",
+                                     "v", "weight", "append_cache", "append_loc"])
+def test_one_host_operand_is_refused(on_host, monkeypatch):
+    """Each operand of the calls above is checked for itself."""
+    lib = _NoLaunch()
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    monkeypatch.setattr(_lib, "raw_stream", lambda device: 0)
+
+    def t(name, *shape, dtype=torch.bfloat16):
+        x = torch.zeros(shape, dtype=dtype)
+        return x if name == on_host else x.as_subclass(_GpuTensor)
+
+    i32 = torch.int32
+    with pytest.raises(ValueError):
+        if on_host in ("page_table", "row_ids"):
+            paged.build_indices(t("page_table", 2, 8, dtype=i32), t("row_ids", 2, dtype=i32),
+                                t("cu_k", 3, dtype=i32), 4)
+        elif on_host == "weight":
+            HipOps().linear(t("x", 3, 128), t("weight", 16, 128))
+        elif on_host.startswith("append"):
+            table = t("cos", 9, 64, dtype=torch.float32)
+            HipOps().qk_norm_rope_append(t("qkv", 3, 8 * 64), t("w", 64), t("w", 64), table, table,
+                                         t("positions", 3, dtype=i32), 4, 1e-6,
+                                         t("append_cache", 4, 2, 64), t("c", 4, 2, 64),
+                                         t("append_loc", 3, dtype=i32))
+        else:
+            paged.bind_kv_append(t("k_cache", 4, 2, 64), t("v_cache", 4, 2, 64),
+                                 t("out_loc", 3, dtype=i32), t("k", 3, 2, 64), t("v", 3, 2, 64))
+    assert lib.calls == []
