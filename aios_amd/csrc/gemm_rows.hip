@@ -48,6 +48,22 @@ __device__ __forceinline__ bf16x8 rows_load(__amdgpu_buffer_rsrc_t r, int voff, 
   return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
 
+// The register steps built for a row tile count, 0 when the K steps per
+// wavefront do not fit, and the steps that every wavefront has of KS
+// (its share is `need` or one less).
+int rows_ks(int mt, int need, bool silu) {
+  if (need <= 3) return 3;
+  if (need <= 4) return 4;
+  if (need <= 6) return silu ? 8 : 6;
+  if (need <= 8) return 8;
+  if (need <= 10) return 10;
+  if (need <= 12 && mt <= 2 && !silu) return 12;
+  return 0;
+}
+constexpr int rows_whole(int ks, bool silu) {
+  return ks == 3 ? 1 : ks == 4 ? 3 : ks == 8 && silu ? 4 : ks - 2;
+}
+
 // NH = 2: a tile's weights in two halves, so that two buffers of KS / 2 steps
 // serve where MT * KS fragments leave no room for two of KS.
 // Register use at two wavefronts per SIMD (256): 4 * (MT * KS + 2 * KS / NH)
@@ -71,7 +87,8 @@ __global__ __launch_bounds__(kRowsThreads) __attribute__((amdgpu_waves_per_eu(2,
   int t = PART ? blockIdx.x / splits : blockIdx.x;
   const int tiles = N / NC;
   // This wavefront's K steps s0 .. s0 + ns - 1 (1 <= ns <= KS: the launcher's
-  // choice of splits); steps past them read x as zero and the last weights.
+  // choice of splits); steps past them read zeros on both sides (weights read
+  // there would meet the zero x, but 0 * Inf is NaN).
   const int T = K >> 5;
   const int unit = split * kRowsWaves + wave, units = (PART ? splits : 1) * kRowsWaves;
   const int s0 = unit * T / units;
@@ -81,9 +98,16 @@ __global__ __launch_bounds__(kRowsThreads) __attribute__((amdgpu_waves_per_eu(2,
   const int wvoff = (wrow * w_stride + lg * 8) * 2;
   const int tile_b = NC * w_stride * 2;
   auto load = [&](bf16x8 (&f)[KH], int tile, int half) {
+    // (the count made opaque for each tile: hoisted out of the loop, the steps'
+    // offsets would take a register each)
+    int n = ns;
+    asm volatile("" : "+s"(n));
 #pragma unroll
-    for (int u = 0; u < KH; ++u)
-      f[u] = rows_load(rw, wvoff, tile * tile_b + (s0 + min(half * KH + u, ns - 1)) * 64);
+    for (int u = 0; u < KH; ++u) {
+      const int step = half * KH + u;
+      const bool pad = step >= rows_whole(KS, SILU) && step >= n;
+      f[u] = rows_load(rw, pad ? kOut : wvoff, tile * tile_b + (s0 + (pad ? 0 : step)) * 64);
+    }
   };
   bf16x8 wa[KH], wb[KH];
   load(wa, t, 0);
@@ -212,18 +236,6 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(const float* __restric
   for (int s = 1; s < kRowsMaxSplits; ++s) o += v[s];
   *reinterpret_cast<uint2*>(y + (int64_t)m * y_stride + n) =
       make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-}
-
-// The register steps built for a row tile count, 0 when the K steps per
-// wavefront do not fit.
-int rows_ks(int mt, int need, bool silu) {
-  if (need <= 3) return 3;
-  if (need <= 4) return 4;
-  if (need <= 6) return silu ? 8 : 6;
-  if (need <= 8) return 8;
-  if (need <= 10) return 10;
-  if (need <= 12 && mt <= 2 && !silu) return 12;
-  return 0;
 }
 
 template <int MT, int KS, int NH = 1>

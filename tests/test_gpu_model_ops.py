@@ -194,6 +194,28 @@ def test_streaming_rows_match_fp32_gemm(m, n, k):
     assert bool(((y - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("m,n,k,silu", [
+    (24, 2560, 4096, False), (24, 2560, 9728, False), (9, 2560, 9728, False), (17, 64, 1280, False),
+    (64, 512, 2304, False), (40, 20016, 2304, False), (3, 48, 1280, False), (17, 64, 1280, True),
+    (64, 512, 2304, True), (40, 10016, 2304, True), (3, 48, 1280, True)])
+def test_infinite_weights_stay_infinite(m, n, k, silu):
+    """Wavefronts and splits whose share of K is a step short of their registers
+    add nothing for it: infinite weights at the end of every K step give the
+    infinity of the plain product, not NaN."""
+    x = _bf16((m, k), m + k, 1.0)
+    x[:, 31::32] = x[:, 31::32].abs() + 0.5
+    w = _bf16((2 * n if silu else n, k), n, 0.05)
+    w[:5, 31::32] = float("inf")
+    if silu:
+        y = HipOps().add_rmsnorm_linear(x, None, torch.ones_like(x[0]), 1e-6, w, silu=True)[0]
+        assert bool(y[:, :5].isinf().all()) and bool(y[:, 8:].isfinite().all())
+    else:
+        w[7, 31::32] = float("-inf")
+        y = HipOps().linear(x, w)
+        assert bool((y[:, :5] == float("inf")).all()) and bool((y[:, 7] == float("-inf")).all())
+        assert bool(y[:, 8:].isfinite().all())
+
+
 @pytest.mark.parametrize("rows,k,n", [(17, 768, 6144), (32, 2560, 512), (9, 2560, 4864),
                                       (24, 1280, 48), (24, 2304, 16), (40, 2560, 256),
                                       (64, 1024, 3072)])
