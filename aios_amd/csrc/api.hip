@@ -36,10 +36,12 @@ constexpr int32_t kMinCascadePrefix = 256;
 // Prefill split, in 32-position sub-tiles (measured on MI355X with both sides
 // of each line; per layer, main launch + combine against one workgroup per
 // tile).
-// Few-row tiles (at most 64 MFMA rows) longer than 6 sub-tiles: 8 tokens of a
-// 32q/8kv x 128 model against 188 positions 8.7 us unsplit and 10.0 split,
-// against 258 positions 11.1 and 10.0, 6 against 4,099 94.7 and 16.2.
-constexpr int32_t kPrefillFewUnsplit = 6;
+// Few-row tiles (at most 64 MFMA rows) longer than 8 sub-tiles: one token of a
+// 32q/8kv x 128 model against 225 positions 9.6 us unsplit and 10.6 split,
+// against 289 11.0 and 10.6 (12q/4kv x 64: 7.7 and 8.5, 8.8 and 8.6), 6
+// against 4,099 94.7 and 16.2; but only while the batch leaves compute units
+// idle (prefill_split_pays).
+constexpr int32_t kPrefillFewUnsplit = 8;
 // Fuller tiles: a part costs about 8 sub-tiles' time (launch, state, merge)
 // and the last part half its length, so a part of 4 sqrt(work per compute
 // unit) sub-tiles balances the two (100 tokens against 4,100 positions: 102
@@ -77,6 +79,34 @@ int device_cus() {
 // against 5.0; 1024 x 2048: 4.4 against 6.0).
 bool rows_form(int64_t rows, int64_t k) {
   return rows > 16 || (k > 1024 && k != 2048 && k != 3072);
+}
+
+// Whether a batch's split beats one workgroup per tile: nanoseconds of both,
+// fitted on MI355X (256 units) to 2,200 batches of 1 to 128 requests, head
+// sizes 64, 96 and 128, 193 to 8,000 positions.  Unsplit, the longest tile is
+// a chain of its sub-tiles.  Few-row parts (at most 64 rows) are one latency
+// chain while there are at most one per unit, then each adds its K/V bytes and
+// its states written and read (96-dim rows are no whole 128-byte lines); fuller
+// parts are a shorter chain, slowed by the work and the workgroups that share
+// its unit.  32q/8kv x 128, 8 tokens each, unsplit / split: 8 requests against
+// 4,099 positions 98.6 / 60 us, 16 against 4,099 99.9 / 107, 32 against 2,000
+// 55.5 / 105, 64 against 1,000 56.6 / 110; 16q/8kv x 128, 3 requests of 1,000
+// tokens and 200 cached: 38.8 / 45.8, one of 2,048: 57 / 42.  The choice is at
+// most 7% slower than the better of the two over those batches.
+bool prefill_split_pays(int32_t head_dim, int32_t rows, int64_t parts, int32_t longest,
+                        int32_t longest_part, int64_t work, int32_t cus) {
+  const int64_t whole = 4000 + 18 * rows + (int64_t)longest * (360 + 14 * head_dim / 5);
+  int64_t split;
+  if (rows <= 64) {
+    const int32_t each = head_dim == 64 ? 1200 : head_dim == 96 ? 1700 : 1900;
+    const int32_t row = head_dim == 64 ? 10 : head_dim == 96 ? 21 : 18;
+    split = 6400 + 33 * head_dim + parts * (each + rows * row) / 100 -
+            8 * (parts < cus ? parts : cus);
+  } else {
+    const int32_t base = head_dim == 64 ? 8000 : head_dim == 96 ? 12000 : 10500;
+    split = base + 300 * longest_part + (5 * work * head_dim / 2 + 5000 * parts) / cus;
+  }
+  return split < whole;
 }
 
 // How a prefill batch splits its tiles' KV ranges over workgroups
@@ -122,6 +152,9 @@ void plan_prefill_parts(aios_attn_plan_t* p, const int32_t* cu_q, const int32_t*
     if (gain < kPrefillMinGain || 2 * gain < part_sub) return;
   }
   const int32_t n = cdiv(longest, part_sub);
+  if (!prefill_split_pays(p->head_dim, rows, count_parts(part_sub), longest, cdiv(longest, n), work,
+                          cus))
+    return;
   const int64_t parts = (int64_t)p->batch_size * p->num_q_tiles * hkv * n;
   const int64_t o_bytes = align_up(parts * rows * p->head_dim * 4, 256);
   const int64_t bytes = n > 1 ? o_bytes + align_up(parts * rows * 8, 256) : 0;

@@ -105,7 +105,7 @@ def test_plan_decode_chunk_length(rows, prefix, hq, hkv, d, chunk):
     assert p.num_parts <= 64
 
 
-@pytest.mark.parametrize("q,kv,hq,hkv,d", [(6, 4099, 32, 8, 128), (1, 193, 8, 8, 64),
+@pytest.mark.parametrize("q,kv,hq,hkv,d", [(6, 4099, 32, 8, 128), (1, 257, 8, 8, 64),
                                           (100, 4100, 32, 8, 128), (2048, 2048, 16, 8, 128),
                                           (4096, 4096, 32, 8, 128), (8, 150, 32, 8, 128)])
 def test_plan_prefill_split(q, kv, hq, hkv, d):
@@ -123,6 +123,26 @@ def test_plan_prefill_split(q, kv, hq, hkv, d):
     rc, small = _plan(_lib.PHASE_PREFILL, [0, q], [0, kv], hq=hq, hkv=hkv, d=d,
                       ws=p.ws_bytes - 1)
     assert rc == 0 and small.num_parts == 0 and small.ws_bytes == 0
+
+
+@pytest.mark.parametrize("reqs,q,kv,hq,hkv,d,split", [
+    # few rows: short ranges (1.2 to 1.6 us a launch slower split), then requests
+    # until their tiles fill the units (1.1 to 2.3 times slower split)
+    (1, 1, 193, 8, 8, 64, False), (1, 8, 256, 32, 8, 128, False), (1, 8, 289, 32, 8, 128, True),
+    (8, 8, 4099, 32, 8, 128, True), (16, 8, 4099, 32, 8, 128, False),
+    (32, 8, 2000, 32, 8, 128, False), (64, 8, 1000, 32, 8, 128, False),
+    (32, 1, 8000, 16, 8, 128, False), (32, 8, 8000, 8, 2, 96, True), (128, 1, 1000, 8, 2, 96, False),
+    (16, 21, 260, 12, 4, 64, False), (32, 1, 8000, 12, 4, 64, True),
+    # fuller tiles: batches whose work is already spread evenly (5 to 19% slower split)
+    (1, 2048, 2048, 16, 8, 128, True), (2, 300, 4099, 32, 8, 128, True),
+    (3, 1000, 1200, 16, 8, 128, False), (3, 300, 1300, 32, 8, 128, False),
+    (6, 400, 900, 8, 2, 96, False), (6, 500, 1500, 12, 4, 64, False),
+])
+def test_plan_prefill_split_of_batches(reqs, q, kv, hq, hkv, d, split):
+    """A batch is split only where the split measured faster."""
+    ramp = np.arange(reqs + 1)
+    rc, p = _plan(_lib.PHASE_PREFILL, q * ramp, kv * ramp, hq=hq, hkv=hkv, d=d, ws=1 << 28)
+    assert rc == 0 and (p.num_parts > 1) == split
 
 
 def test_plan_rejects_bad_batches():
