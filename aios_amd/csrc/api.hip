@@ -91,17 +91,17 @@ bool rows_form(int64_t rows, int64_t k) {
 // its unit.  32q/8kv x 128, 8 tokens each, unsplit / split: 8 requests against
 // 4,099 positions 98.6 / 60 us, 16 against 4,099 99.9 / 107, 32 against 2,000
 // 55.5 / 105, 64 against 1,000 56.6 / 110; 16q/8kv x 128, 3 requests of 1,000
-// tokens and 200 cached: 38.8 / 45.8, one of 2,048: 57 / 42.  The choice is at
-// most 7% slower than the better of the two over those batches.
+// tokens and 200 cached: 38.8 / 45.8, one of 2,048: 57 / 42.  Over those
+// batches the choice is at most 8% slower than unsplit and 10% than split.
 bool prefill_split_pays(int32_t head_dim, int32_t rows, int64_t parts, int32_t longest,
                         int32_t longest_part, int64_t work, int32_t cus) {
   const int64_t whole = 4000 + 18 * rows + (int64_t)longest * (360 + 14 * head_dim / 5);
   int64_t split;
   if (rows <= 64) {
-    const int32_t each = head_dim == 64 ? 1200 : head_dim == 96 ? 1700 : 1900;
-    const int32_t row = head_dim == 64 ? 10 : head_dim == 96 ? 21 : 18;
-    split = 6400 + 33 * head_dim + parts * (each + rows * row) / 100 -
-            8 * (parts < cus ? parts : cus);
+    const int32_t base = head_dim == 64 ? 8900 : head_dim == 96 ? 9900 : 10200;
+    const int32_t each = head_dim == 64 ? 1300 : 1700;
+    const int32_t row = head_dim == 64 ? 10 : head_dim == 96 ? 24 : 18;
+    split = base + parts * (each + rows * row) / 100 - 12 * (parts < cus ? parts : cus);
   } else {
     const int32_t base = head_dim == 64 ? 8000 : head_dim == 96 ? 12000 : 10500;
     split = base + 300 * longest_part + (5 * work * head_dim / 2 + 5000 * parts) / cus;

@@ -124,8 +124,8 @@ def test_growing_logits_move_the_softmax_reference(q_lens, kv_lens, hq, hkv, d):
 
 
 @pytest.mark.parametrize("q_lens,kv_lens,hq,hkv,d", [
-    ([1], [257], 8, 8, 64),                    # few rows: the shortest split range, one row
-                                               # (up to 256 positions one workgroup is faster)
+    ([1], [289], 8, 8, 64),                    # few rows: the shortest split range, one row
+                                               # (up to 288 positions one workgroup is faster)
     ([8], [513], 32, 8, 128),                  # one full 32-row tile, one position over a part
     ([9], [1000], 32, 8, 128),                 # 36 rows: two row tiles, half the wavefronts each
     ([16, 1, 3], [900, 300, 40], 8, 2, 96),    # ragged few-row batch, one tile unsplit

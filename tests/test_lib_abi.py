@@ -105,7 +105,7 @@ def test_plan_decode_chunk_length(rows, prefix, hq, hkv, d, chunk):
     assert p.num_parts <= 64
 
 
-@pytest.mark.parametrize("q,kv,hq,hkv,d", [(6, 4099, 32, 8, 128), (1, 257, 8, 8, 64),
+@pytest.mark.parametrize("q,kv,hq,hkv,d", [(6, 4099, 32, 8, 128), (1, 289, 8, 8, 64),
                                           (100, 4100, 32, 8, 128), (2048, 2048, 16, 8, 128),
                                           (4096, 4096, 32, 8, 128), (8, 150, 32, 8, 128)])
 def test_plan_prefill_split(q, kv, hq, hkv, d):
