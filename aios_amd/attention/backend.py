@@ -36,7 +36,7 @@ from typing import TYPE_CHECKING
 import torch
 
 from aios_amd import _lib, paged
-from aios_amd.core import get_global_ctx
+from aios_amd.core import get_global_ctx, runs_as_built
 from aios_amd.kvcache import MHAKVCache
 
 from .base import BaseAttentionBackend, BaseAttentionMetadata
@@ -155,6 +155,10 @@ def check_decode_preconditions(indices: torch.Tensor, cu_seqlens_k: torch.Tensor
         last = indices[cu[1:] - 1]
         if not bool((out_loc.to(last.dtype) == last).all()):
             raise ValueError("out_loc[b] must be row b's last page id (Batch.fused_append)")
+
+
+# What the one-launch append stands for, as this package defines it.
+_POOL = {name: getattr(MHAKVCache, name) for name in ("store_kv", "k_cache", "v_cache")}
 
 
 class Mi355xAttentionBackend(BaseAttentionBackend):
@@ -498,9 +502,7 @@ class Mi355xAttentionBackend(BaseAttentionBackend):
         batches go through store_kv, with its conversions and errors."""
         if not batch.is_prefill or not isinstance(batch.attn_metadata, Mi355xAttentionMetadata):
             return False
-        if (type(self).forward is not Mi355xAttentionBackend.forward or "forward" in vars(self)
-                or type(paged_kv_cache).store_kv is not MHAKVCache.store_kv
-                or "store_kv" in vars(paged_kv_cache)):
+        if not (runs_as_built(self, _FORWARD) and runs_as_built(paged_kv_cache, _POOL)):
             return False  # (a caller's own forward or store_kv sees every call)
         loc = batch.out_loc
         return (paged_kv_cache.row_shape == (self.num_kv_heads, self.head_dim)
@@ -560,3 +562,6 @@ class Mi355xAttentionBackend(BaseAttentionBackend):
                            v_cache.view(-1, self.num_kv_heads, self.head_dim), metadata.indices,
                            metadata.cu_seqlens_k_gpu, workspace=ws, sm_scale=self.sm_scale)
         return out.reshape(bsz, -1)
+
+
+_FORWARD = {name: getattr(Mi355xAttentionBackend, name) for name in ("forward", "_prefill")}

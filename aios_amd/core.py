@@ -148,3 +148,12 @@ def reset_global_ctx() -> None:
     """Drop the process-global context (tests and benches build several)."""
     global _GLOBAL_CTX
     _GLOBAL_CTX = None
+
+
+def runs_as_built(obj, calls: dict) -> bool:
+    """Whether ``obj``'s methods named in ``calls`` are those functions: not
+    overridden by its class, set on the object or reached through a wrapper,
+    so that a launch which stands for them passes no call of the caller's by."""
+    own = getattr(obj, "__dict__", ())
+    return all(getattr(type(obj), name, None) is fn and name not in own
+               for name, fn in calls.items())

@@ -20,7 +20,11 @@ import torch.nn.functional as F
 
 from aios_amd.attention import BaseAttentionBackend, Mi355xAttentionBackend
 from aios_amd.config import ModelConfig
-from aios_amd.core import get_global_ctx
+from aios_amd.core import get_global_ctx, runs_as_built
+from aios_amd.layers import HipOps
+
+# The op that qk_norm_rope_append stands for, as this package defines it.
+_ROPE = {"qk_norm_rope": HipOps.qk_norm_rope}
 
 
 def init_weights(config: ModelConfig, seed: int, device="cpu",
@@ -105,11 +109,7 @@ class Qwen3ForCausalLM:
         self.device = torch.device(device)
         self.w = weights
         self.attn_backend = attn_backend or Mi355xAttentionBackend(config)
-        if ops is None:
-            from aios_amd.layers import HipOps
-
-            ops = HipOps()
-        self.ops = ops
+        self.ops = HipOps() if ops is None else ops
         self.rotary = RotaryEmbedding(config.head_dim,
                                       max_positions or min(config.max_position_embeddings, 8192),
                                       config.rope_theta, self.device)
@@ -144,8 +144,8 @@ class Qwen3ForCausalLM:
             out = be.forward_rope(q, k, v, lw["q_norm"], lw["k_norm"], self.rotary.cos_bf16,
                                   self.rotary.sin_bf16, positions, c.rms_norm_eps, kv_cache, i,
                                   batch)
-        elif (getattr(self.ops, "rope_in_append", False)
-                and getattr(be, "append_rope_applies", None) is not None
+        elif (getattr(self.ops, "rope_in_append", False) and runs_as_built(self.ops, _ROPE)
+                and issubclass(type(be), Mi355xAttentionBackend)
                 and be.append_rope_applies(qkv, kv_cache, batch)):
             k_cache, v_cache = be.layer_kv(kv_cache, i)
             q = self.ops.qk_norm_rope_append(qkv, lw["q_norm"], lw["k_norm"], self.rotary.cos,
