@@ -92,6 +92,13 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
 // wavefronts w and w + 2 take the two halves of row tile w, and the states
 // of a row tile are merged through the ring once every sub-tile is consumed.
 
+// The parts of a tile of `rows` MFMA rows over kv positions: one, written
+// directly, where it has more rows than the plan gave each part room for
+// (lengths on the device other than the planned ones).
+__device__ __forceinline__ PrefillParts tile_parts(const PrefillArgs& a, int rows, int kv) {
+  return prefill_parts(kv, a.part_sub, rows <= a.part_rows ? a.n_parts : 1);
+}
+
 // Dims 8 dg .. 8 dg + 7 of row m in a part's o.
 template <int D>
 __device__ __forceinline__ int64_t prefill_part_o(const PrefillArgs& a, int64_t part, int dg, int m) {
@@ -125,14 +132,13 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
   const int cached = kv_len - q_len;
   const int q_hi = min(q_len, (qt + 1) * a.q_tile);
   const int kv_hi = min(kv_len, cached + q_hi);
-  const PrefillParts pp = prefill_parts(kv_hi, a.part_sub, a.n_parts);
+  const int rows = (q_hi - qt * a.q_tile) * G;
+  const PrefillParts pp = tile_parts(a, rows, kv_hi);
   if (s >= pp.n) return;
   const int kv_begin = s * pp.per * kSubTok;
   const int kv_end = min(kv_hi, kv_begin + pp.per * kSubTok);
 
   // Wavefront -> (row tile, share of the sub-tiles).
-  // (at most what the plan gave each part room for)
-  const int rows = min((q_hi - qt * a.q_tile) * G, a.part_rows);
   const int nr = rows <= 32 ? 1 : rows <= 64 ? 2 : 4;
   const int rt = wave & (nr - 1);
   const int share = nr == 4 ? 0 : nr == 2 ? wave >> 1 : wave;
@@ -275,9 +281,8 @@ __global__ __launch_bounds__(NW * 64) void prefill_combine_kernel(PrefillArgs a,
   if (qt * a.q_tile >= q_len) return;
   const int kv_len = a.cu_k[r + 1] - a.cu_k[r];
   const int q_hi = min(q_len, (qt + 1) * a.q_tile);
-  const PrefillParts pp =
-      prefill_parts(min(kv_len, kv_len - q_len + q_hi), a.part_sub, a.n_parts);
-  const int rows = min((q_hi - qt * a.q_tile) * a.group, a.part_rows);
+  const int rows = (q_hi - qt * a.q_tile) * a.group;
+  const PrefillParts pp = tile_parts(a, rows, min(kv_len, kv_len - q_len + q_hi));
   if (pp.n == 1 || rb * RB >= rows) return;  // (uniform)
   const int dg = lane % DG;
   const int m = rb * RB + lane / DG;

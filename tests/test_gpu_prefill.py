@@ -163,3 +163,19 @@ def test_split_kv_ranges_match_oracle(q_lens, kv_lens, hq, hkv, d):
     out = paged.prefill(small, q.to(DEV), kc.to(DEV), vc.to(DEV), idx.to(DEV), cu_q.to(DEV),
                         cu_k.to(DEV))
     np.testing.assert_allclose(to_np64(out), ref, **BF16_TOL)
+
+
+@pytest.mark.parametrize("planned,q_lens,kv_lens,hq,hkv,d", [
+    ([2, 2], [1, 3], [600, 600], 8, 2, 96),      # 12 rows in parts made for 8
+    ([8, 8], [1, 15], [900, 700], 32, 8, 128),   # 60 rows in parts made for 32
+    ([20, 20], [30, 10], [900, 1100], 8, 2, 64), # 120 rows in parts made for 80
+])
+def test_tiles_fuller_than_planned(planned, q_lens, kv_lens, hq, hkv, d):
+    # The lengths on the device put more rows in a tile than the plan's parts
+    # have room for: that tile is computed whole, as without the split.
+    q, kc, vc, idx, cu_q, cu_k = _make(q_lens, kv_lens, hq, hkv, d, 4096, seed=sum(kv_lens))
+    p = paged.plan("prefill", [0, planned[0], sum(planned)], cu_k, hq, hkv, d)
+    assert p.num_parts > 1 and p.max_q_len < max(q_lens)
+    out = paged.prefill(p, q.to(DEV), kc.to(DEV), vc.to(DEV), idx.to(DEV), cu_q.to(DEV),
+                        cu_k.to(DEV))
+    np.testing.assert_allclose(to_np64(out), _oracle(q, kc, vc, idx, cu_q, cu_k, d), **BF16_TOL)
