@@ -422,11 +422,10 @@ int aios_attn_prefill_ws(const aios_attn_plan_t* p, const void* q, int64_t q_tok
   a.q_tiles = p->num_q_tiles;
   a.batch = p->batch_size;
   a.out = static_cast<aios::bf16*>(out);
-  // Split tiles need room for their partial states; without it (or with a
-  // plan that has none) each tile is one workgroup.
-  if (p->num_parts > 0 && (p->ws_bytes == 0 || (workspace && p->ws_bytes <= workspace_bytes))) {
-    if (((uintptr_t)workspace & 255) != 0)
-      return fail(AIOS_ERR_INVALID, "prefill: workspace must be 256-byte aligned");
+  // Split tiles need room for their partial states, 256-byte aligned; without
+  // it (or with a plan that has none) each tile is one workgroup.
+  if (p->num_parts > 1 && workspace && ((uintptr_t)workspace & 255) == 0 &&
+      p->ws_bytes <= workspace_bytes) {
     char* ws = static_cast<char*>(workspace);
     a.part_sub = p->prefix_chunk_len / 32;
     a.n_parts = p->num_parts;

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from aios_amd import paged
+from aios_amd import _lib, paged
 from oracle import attention as oatt
 from tests.util import BF16_TOL, to_np64
 
@@ -179,3 +179,19 @@ def test_tiles_fuller_than_planned(planned, q_lens, kv_lens, hq, hkv, d):
     out = paged.prefill(p, q.to(DEV), kc.to(DEV), vc.to(DEV), idx.to(DEV), cu_q.to(DEV),
                         cu_k.to(DEV))
     np.testing.assert_allclose(to_np64(out), _oracle(q, kc, vc, idx, cu_q, cu_k, d), **BF16_TOL)
+
+
+def test_unaligned_workspace_runs_unsplit():
+    q, kc, vc, idx, cu_q, cu_k = _make([6], [900], 8, 2, 96, 4096, seed=5)
+    p = paged.plan("prefill", cu_q, cu_k, 8, 2, 96)
+    assert p.num_parts > 1
+    on = [t.to(DEV) for t in (q, kc, vc, idx, cu_q, cu_k)]
+    ws = torch.full((p.ws_bytes + 256,), 85, dtype=torch.uint8, device=DEV)
+    out = torch.empty_like(on[0])
+    _lib.check(_lib.lib().aios_attn_prefill_ws(
+        p, on[0].data_ptr(), on[0].stride(0), on[1].data_ptr(), on[2].data_ptr(), kc.shape[0],
+        on[3].data_ptr(), on[4].data_ptr(), on[5].data_ptr(), out.data_ptr(), ws.data_ptr() + 64,
+        p.ws_bytes, 96 ** -0.5, 0), "prefill")
+    torch.cuda.synchronize()
+    assert bool((ws == 85).all())
+    np.testing.assert_allclose(to_np64(out), _oracle(q, kc, vc, idx, cu_q, cu_k, 96), **BF16_TOL)
