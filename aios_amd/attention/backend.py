@@ -158,7 +158,7 @@ def check_decode_preconditions(indices: torch.Tensor, cu_seqlens_k: torch.Tensor
 
 
 # What the one-launch append stands for, as this package defines it.
-_POOL = {name: getattr(MHAKVCache, name) for name in ("store_kv", "k_cache", "v_cache")}
+_POOL = tuple((name, getattr(MHAKVCache, name)) for name in ("store_kv", "k_cache", "v_cache"))
 
 
 class Mi355xAttentionBackend(BaseAttentionBackend):
@@ -564,4 +564,4 @@ class Mi355xAttentionBackend(BaseAttentionBackend):
         return out.reshape(bsz, -1)
 
 
-_FORWARD = {name: getattr(Mi355xAttentionBackend, name) for name in ("forward", "_prefill")}
+_FORWARD = tuple((name, getattr(Mi355xAttentionBackend, name)) for name in ("forward", "_prefill"))

@@ -150,10 +150,13 @@ def reset_global_ctx() -> None:
     _GLOBAL_CTX = None
 
 
-def runs_as_built(obj, calls: dict) -> bool:
-    """Whether ``obj``'s methods named in ``calls`` are those functions: not
-    overridden by its class, set on the object or reached through a wrapper,
-    so that a launch which stands for them passes no call of the caller's by."""
-    own = getattr(obj, "__dict__", ())
-    return all(getattr(type(obj), name, None) is fn and name not in own
-               for name, fn in calls.items())
+def runs_as_built(obj, calls: tuple) -> bool:
+    """Whether ``obj``'s methods, (name, function) in ``calls``, are those
+    functions: not overridden by its class, set on the object or reached
+    through a wrapper, so that a launch which stands for them passes no call
+    of the caller's by."""
+    cls, own = type(obj), getattr(obj, "__dict__", ())
+    for name, fn in calls:
+        if getattr(cls, name, None) is not fn or name in own:
+            return False
+    return True

@@ -24,7 +24,7 @@ from aios_amd.core import get_global_ctx, runs_as_built
 from aios_amd.layers import HipOps
 
 # The op that qk_norm_rope_append stands for, as this package defines it.
-_ROPE = {"qk_norm_rope": HipOps.qk_norm_rope}
+_ROPE = (("qk_norm_rope", HipOps.qk_norm_rope),)
 
 
 def init_weights(config: ModelConfig, seed: int, device="cpu",
@@ -134,13 +134,13 @@ class Qwen3ForCausalLM:
         lw = self.w["layers"][i]
         t = qkv.shape[0]
         hq, hkv, d = c.num_qo_heads, c.num_kv_heads, c.head_dim
-        v = qkv[:, self._q_size + self._kv_size:].view(t, hkv, d)
         be = self.attn_backend
         if (getattr(self.ops, "rope_in_decode", False)
                 and getattr(be, "decode_rope_applies", None) is not None
                 and be.decode_rope_applies(batch)):
             q = qkv[:, :self._q_size].view(t, hq, d)
             k = qkv[:, self._q_size:self._q_size + self._kv_size].view(t, hkv, d)
+            v = qkv[:, self._q_size + self._kv_size:].view(t, hkv, d)
             out = be.forward_rope(q, k, v, lw["q_norm"], lw["k_norm"], self.rotary.cos_bf16,
                                   self.rotary.sin_bf16, positions, c.rms_norm_eps, kv_cache, i,
                                   batch)
@@ -153,6 +153,7 @@ class Qwen3ForCausalLM:
                                              k_cache, v_cache, batch.out_loc.view(-1))
             out = be.prefill_appended(q, k_cache, v_cache, batch)
         else:
+            v = qkv[:, self._q_size + self._kv_size:].view(t, hkv, d)
             q, k = self.ops.qk_norm_rope(qkv, lw["q_norm"], lw["k_norm"], self.rotary.cos,
                                          self.rotary.sin, positions, hq, hkv, d, c.rms_norm_eps)
             out = be.forward(q, k, v, kv_cache, i, batch)

@@ -221,6 +221,7 @@ def _host_calls():
         "build_indices": lambda: paged.build_indices(i32(2, 8), i32(2), i32(3), 4),
         "bind_kv_append": lambda: paged.bind_kv_append(cache, cache, i32(3), kv, kv)(),
         "raw_stream": lambda: _lib.raw_stream(torch.device("cpu")),
+        "raw_stream_indexed": lambda: _lib.raw_stream(torch.device("cpu", 0)),
         "raw_stream_meta": lambda: _lib.raw_stream(torch.device("meta")),
     }
 
