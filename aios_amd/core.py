@@ -15,6 +15,8 @@ that guarantee what they state (the CandidateGroup engine here):
 """
 from __future__ import annotations
 
+import gc
+import threading
 from contextlib import contextmanager
 from dataclasses import dataclass, field
 from typing import TYPE_CHECKING, List, Literal, Optional
@@ -160,3 +162,25 @@ def runs_as_built(obj, calls: tuple) -> bool:
         if getattr(cls, name, None) is not fn or name in own:
             return False
     return True
+
+
+_capture_lock = threading.Lock()
+_captures: list[bool] = []  # of the captures under way: was the collector on before the first
+
+
+@contextmanager
+def captured(graph: torch.cuda.CUDAGraph, stream: torch.cuda.Stream):
+    """torch.cuda.graph with Python's cycle collector held off.  A collection
+    inside a capture would destroy the graphs that dropped reference cycles
+    still hold (an engine let go, say), whose release is not permitted while a
+    stream captures and ends the process."""
+    with _capture_lock:
+        _captures.append(_captures[0] if _captures else gc.isenabled())
+        gc.disable()
+    try:
+        with torch.cuda.graph(graph, stream=stream):
+            yield
+    finally:
+        with _capture_lock:
+            if _captures.pop() and not _captures:
+                gc.enable()

@@ -40,7 +40,8 @@ import torch
 
 from aios_amd import _lib
 from aios_amd.config import ModelConfig
-from aios_amd.core import Batch, Context, Req, SamplingParams, reset_global_ctx, set_global_ctx
+from aios_amd.core import (Batch, Context, Req, SamplingParams, captured, reset_global_ctx,
+                           set_global_ctx)
 from aios_amd.sample import sample_step, stateless_uniforms
 from aios_amd.kvcache import MHAKVCache
 from aios_amd.paged import greedy_select
@@ -731,7 +732,7 @@ class _PrefillGraph:
         with torch.cuda.stream(stream):
             out = self._body()
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=stream):
+        with captured(graph, stream):
             self.logits = self._body()
         cur.wait_stream(stream)
         self.graph = graph
@@ -918,7 +919,7 @@ class _DecodeGraph:
         with torch.cuda.stream(stream):
             self._body()
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=stream):
+        with captured(graph, stream):
             self._body()
         cur.wait_stream(stream)
         self.graph = graph

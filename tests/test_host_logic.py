@@ -2,10 +2,14 @@
 selection and the engine's argument checks (CPU only)."""
 from __future__ import annotations
 
+import contextlib
+import gc
+from types import SimpleNamespace
+
 import pytest
 import torch
 
-from aios_amd import _lib, paged
+from aios_amd import _lib, ime, paged
 from aios_amd.core import Req, SamplingParams
 from aios_amd.ime import (Candidate, CandidateGroupConfig, adaptive_refill_attempts,
                            candidate_valid, select_top, token_longest_common_prefix)
@@ -274,3 +278,53 @@ def test_one_host_operand_is_refused(on_host, monkeypatch):
             paged.bind_kv_append(t("k_cache", 4, 2, 64), t("v_cache", 4, 2, 64),
                                  t("out_loc", 3, dtype=i32), t("k", 3, 2, 64), t("v", 3, 2, 64))
     assert lib.calls == []
+
+
+@pytest.mark.parametrize("kind", ["decode", "prefill"])
+@pytest.mark.parametrize("enabled", [True, False])
+@pytest.mark.parametrize("fails", [False, True])
+def test_captures_hold_the_collector_off(kind, enabled, fails, monkeypatch):
+    """A graph that a dropped reference cycle still holds must not be destroyed
+    (by Python's cycle collector) while another one is being captured: the
+    collector is off from capture_begin to capture_end, and as before after."""
+    seen = []
+
+    @contextlib.contextmanager
+    def capture(graph, stream=None):
+        seen.append(gc.isenabled())
+        try:
+            yield
+        finally:
+            seen.append(gc.isenabled())
+
+    stream = SimpleNamespace(wait_stream=lambda s: None)
+    monkeypatch.setattr(torch.cuda, "graph", capture)
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda: SimpleNamespace(replay=lambda: None))
+    monkeypatch.setattr(torch.cuda, "Stream", lambda dev: stream)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev: stream)
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+    cls = ime._DecodeGraph if kind == "decode" else ime._PrefillGraph
+    g = cls.__new__(cls)
+    g.rt, g.graph, calls = SimpleNamespace(device="cuda"), None, []
+
+    def body():
+        calls.append(gc.isenabled())
+        if fails and len(calls) == 2:
+            raise RuntimeError("no room")
+
+    g._body = body
+    if kind == "prefill":
+        g.q_len = 1
+        g.ids = g.pos = g.out_loc = torch.zeros(1, dtype=torch.long)
+        g.ramp = g.kv_len = torch.zeros(1, dtype=torch.long)
+    run = g.run_step if kind == "decode" else lambda: g.run([5], 0, torch.zeros(1))
+    was = gc.isenabled()
+    try:
+        gc.enable() if enabled else gc.disable()
+        with pytest.raises(RuntimeError) if fails else contextlib.nullcontext():
+            run()
+        assert gc.isenabled() == enabled
+    finally:
+        gc.enable() if was else gc.disable()
+    assert calls == [enabled, False] and seen == [False, False]
+    assert (g.graph is None) == fails
