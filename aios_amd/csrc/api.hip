@@ -743,7 +743,7 @@ int aios_qk_norm_rope(const void* qkv, int64_t qkv_stride, int64_t tokens, int32
     return fail(AIOS_ERR_INVALID, "qk_norm_rope: rows must be 4-byte aligned");
   return check_hip(aios::qk_norm_rope(qkv, qkv_stride, tokens, num_qo_heads, num_kv_heads, head_dim,
                                       q_weight, k_weight, cos_table, sin_table, table_rows,
-                                      positions, q_out, k_out, eps, nullptr, 0, nullptr,
+                                      positions, q_out, k_out, eps,
                                       static_cast<hipStream_t>(stream)),
                    "qk_norm_rope launch");
 }
@@ -767,10 +767,11 @@ int aios_qk_norm_rope_append(const void* qkv, int64_t qkv_stride, int64_t tokens
   if ((((uintptr_t)qkv | (uintptr_t)q_weight | (uintptr_t)k_weight | (uintptr_t)k_cache |
         (uintptr_t)v_cache) & 3) != 0)
     return fail(AIOS_ERR_INVALID, "qk_norm_rope_append: rows must be 4-byte aligned");
-  return check_hip(aios::qk_norm_rope(qkv, qkv_stride, tokens, num_qo_heads, num_kv_heads, head_dim,
-                                      q_weight, k_weight, cos_table, sin_table, table_rows,
-                                      positions, q_out, k_cache, eps, v_cache, num_slots, out_loc,
-                                      static_cast<hipStream_t>(stream)),
+  return check_hip(aios::qk_norm_rope_append(qkv, qkv_stride, tokens, num_qo_heads, num_kv_heads,
+                                             head_dim, q_weight, k_weight, cos_table, sin_table,
+                                             table_rows, positions, q_out, k_cache, v_cache,
+                                             num_slots, out_loc, eps,
+                                             static_cast<hipStream_t>(stream)),
                    "qk_norm_rope_append launch");
 }
 

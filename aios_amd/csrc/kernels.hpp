@@ -148,13 +148,17 @@ hipError_t rmsnorm(const void* x, int64_t x_stride, const void* residual, int64_
                    int64_t out_stride, int64_t rows, int hidden, float eps, hipStream_t stream);
 bool rmsnorm_supported(int hidden);
 
-// v_out not null (the append form): k_out / v_out are the [num_slots][hkv][D]
-// caches, written at out_loc[t].
 hipError_t qk_norm_rope(const void* qkv, int64_t stride, int64_t tokens, int hq, int hkv, int D,
                         const void* qw, const void* kw, const float* cos_t, const float* sin_t,
                         int64_t table_rows, const int32_t* positions, void* q_out, void* k_out,
-                        float eps, void* v_out, int64_t num_slots, const int32_t* out_loc,
-                        hipStream_t stream);
+                        float eps, hipStream_t stream);
+// The same with K and V rows written to rows out_loc[t] of the
+// [num_slots][hkv][D] caches.
+hipError_t qk_norm_rope_append(const void* qkv, int64_t stride, int64_t tokens, int hq, int hkv, int D,
+                               const void* qw, const void* kw, const float* cos_t,
+                               const float* sin_t, int64_t table_rows, const int32_t* positions,
+                               void* q_out, void* k_cache, void* v_cache, int64_t num_slots,
+                               const int32_t* out_loc, float eps, hipStream_t stream);
 
 hipError_t silu_mul(const void* x, int64_t x_stride, int64_t rows, int inter, void* out,
                     int64_t out_stride, hipStream_t stream);

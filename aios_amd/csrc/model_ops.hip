@@ -83,42 +83,91 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(
   }
 }
 
-// One wavefront per token and 4 GPW heads (one 16-lane row per head, GPW
-// groups of four); lane l16 of a row holds dims [l16*E, l16*E + E) with
-// E = D/16, so dim i and its rotation partner i +- D/2 sit in lanes l16 and
-// l16 ^ 8.  A lane's cos / sin entries are the same for every head of its
-// token: with many tokens a wavefront takes several groups and reads them
-// once (the fp32 tables are four times a head's bytes), with few tokens one
-// group each, for the parallelism.
-//
-// APPEND (a prefill): the K rows go straight to their pages k_cache[out_loc[t]]
-// and hkv more heads per token copy the V rows to v_cache[out_loc[t]] (slots
-// outside [0, num_slots) are skipped), which is the separate KV append without
-// its launch and its second pass over K.  Measured per layer (traced; rope +
-// append launches -> one): 6 tokens of 32q/8kv x 128 5.0 + 4.5 -> 4.1 us;
-// 2,048 of 16q/8kv x 128 8.2 + 5.0 -> 10.4 us (one group per wavefront 11.4).
-constexpr int kQkWaves = 4;  // wavefronts per workgroup
-
-template <int D, bool APPEND, int GPW>
-__global__ __launch_bounds__(kQkWaves * 64) void qk_norm_rope_kernel(
-    const bf16* __restrict__ qkv, int64_t stride, int64_t tokens, int hq, int hkv,
-    const bf16* __restrict__ qw, const bf16* __restrict__ kw, const float* __restrict__ cos_t,
+// One wavefront per token and four heads (one 16-lane row per head); lane
+// l16 of a row holds dims [l16*E, l16*E + E) with E = D/16, so dim i and its
+// rotation partner i +- D/2 sit in lanes l16 and l16 ^ 8.
+template <int D>
+__global__ __launch_bounds__(64) void qk_norm_rope_kernel(
+    const bf16* __restrict__ qkv, int64_t stride, int hq, int hkv, const bf16* __restrict__ qw,
+    const bf16* __restrict__ kw, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, int64_t table_rows, const int32_t* __restrict__ positions,
-    bf16* __restrict__ q_out, bf16* __restrict__ k_out, float eps, bf16* __restrict__ v_out,
-    int64_t num_slots, const int32_t* __restrict__ out_loc) {
+    bf16* __restrict__ q_out, bf16* __restrict__ k_out, float eps) {
   constexpr int E = D / 16;
-  constexpr int W = E / 2;  // 32-bit words per lane
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x;
   const int l16 = lane & 15;
-  const int heads = hq + (APPEND ? 2 : 1) * hkv;
-  const int sets = (heads + 4 * GPW - 1) / (4 * GPW);
-  const int64_t unit = (int64_t)blockIdx.x * kQkWaves + (threadIdx.x >> 6);
-  const int64_t t = unit / sets;
-  if (t >= tokens) return;
-  const int head0 = (int)(unit - t * sets) * 4 * GPW + (lane >> 4);
+  const int head = blockIdx.y * 4 + (lane >> 4);
+  const int64_t t = blockIdx.x;
+  if (head >= hq + hkv) return;
+  const bool is_q = head < hq;
+  const int hh = is_q ? head : head - hq;
+  const bf16* src = qkv + t * stride + (is_q ? 0 : (int64_t)hq * D) + (int64_t)hh * D + l16 * E;
+  const bf16* wp = (is_q ? qw : kw) + l16 * E;
+  float x[E], wv[E];
+#pragma unroll
+  for (int i = 0; i < E; i += 2) {
+    const uint32_t a = *reinterpret_cast<const uint32_t*>(src + i);
+    const uint32_t b = *reinterpret_cast<const uint32_t*>(wp + i);
+    x[i] = lo_bf16(a);
+    x[i + 1] = hi_bf16(a);
+    wv[i] = lo_bf16(b);
+    wv[i + 1] = hi_bf16(b);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < E; ++i) ss = fmaf(x[i], x[i], ss);
+  const float inv = rsqrtf(row16_sum(ss) / (float)D + eps);
+  float xn[E], pn[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) xn[i] = round_bf16(x[i] * inv * wv[i]);
+#pragma unroll
+  for (int i = 0; i < E; ++i) pn[i] = __shfl_xor(xn[i], 8);
   // Positions outside the table are clamped (never read out of bounds).
   const int64_t pos = min(max((int64_t)positions[t], (int64_t)0), table_rows - 1);
-  const int64_t slot = APPEND ? (int64_t)out_loc[t] : 0;
+  const float* cr = cos_t + pos * D + l16 * E;
+  const float* sr = sin_t + pos * D + l16 * E;
+  const bool first_half = l16 < 8;
+  float y[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const float c = round_bf16(cr[i]);
+    const float s = round_bf16(sr[i]);
+    const float rot = first_half ? -pn[i] : pn[i];
+    y[i] = round_bf16(round_bf16(xn[i] * c) + round_bf16(rot * s));
+  }
+  bf16* dst = (is_q ? q_out + (t * hq + hh) * D : k_out + (t * hkv + hh) * D) + l16 * E;
+#pragma unroll
+  for (int i = 0; i < E; i += 2)
+    *reinterpret_cast<uint32_t*>(dst + i) = pack_bf16x2(y[i], y[i + 1]);
+}
+
+// The same for a prefill, the K rows written straight to their pages
+// k_cache[out_loc[t]] and hkv more heads per token copying the V rows to
+// v_cache[out_loc[t]] (slots outside [0, num_slots) are skipped): the separate
+// KV append without its launch and its second pass over K.  A lane's cos / sin
+// entries are the same for every head of its token: with many tokens a
+// wavefront takes GPW groups of four heads and reads them once (the fp32 tables
+// are four times a head's bytes), with few tokens one group each, for the
+// parallelism.  Per launch in a graph, a 2-D grid against workgroups of four
+// wavefronts that divided their index by the head sets: 6 tokens of 32q/8kv x
+// 128 2.58 -> 2.37 us, 2,048 of 16q/8kv x 128 10.0 -> 9.4 (traced, with the
+// two launches it stands for 5.0 + 4.5 -> 4.1 and 8.2 + 5.0 -> 10.4).
+template <int D, int GPW>
+__global__ __launch_bounds__(64) void qk_norm_rope_append_kernel(
+    const bf16* __restrict__ qkv, int64_t stride, int hq, int hkv, const bf16* __restrict__ qw,
+    const bf16* __restrict__ kw, const float* __restrict__ cos_t,
+    const float* __restrict__ sin_t, int64_t table_rows, const int32_t* __restrict__ positions,
+    bf16* __restrict__ q_out, bf16* __restrict__ k_cache, bf16* __restrict__ v_cache,
+    int64_t num_slots, const int32_t* __restrict__ out_loc, float eps) {
+  constexpr int E = D / 16;
+  constexpr int W = E / 2;  // 32-bit words per lane
+  const int lane = threadIdx.x;
+  const int l16 = lane & 15;
+  const int heads = hq + 2 * hkv;
+  const int head0 = blockIdx.y * 4 * GPW + (lane >> 4);
+  const int64_t t = blockIdx.x;
+  // Positions outside the table are clamped (never read out of bounds).
+  const int64_t pos = min(max((int64_t)positions[t], (int64_t)0), table_rows - 1);
+  const int64_t slot = out_loc[t];
   // (the head's row in qkv; heads past the last one read it and store nothing)
   uint32_t x[GPW][W];
 #pragma unroll
@@ -136,21 +185,19 @@ __global__ __launch_bounds__(kQkWaves * 64) void qk_norm_rope_kernel(
     s[i] = round_bf16(sr[i]);
   }
   const bool first_half = l16 < 8;
-  const bool slot_ok = !APPEND || (slot >= 0 && slot < num_slots);
+  const bool slot_ok = slot >= 0 && slot < num_slots;
 #pragma unroll
   for (int g = 0; g < GPW; ++g) {
     const int head = head0 + 4 * g;
     const bool is_q = head < hq;
     const int hh = is_q ? head : head - hq;
-    if constexpr (APPEND) {
-      if (__ballot(is_q || hh < hkv) == 0) {  // four V heads (or none): copied
-        if (head < heads && slot_ok) {
-          uint32_t* dst = reinterpret_cast<uint32_t*>(v_out + (slot * hkv + hh - hkv) * D + l16 * E);
+    if (__ballot(is_q || hh < hkv) == 0) {  // four V heads (or none): copied
+      if (head < heads && slot_ok) {
+        uint32_t* dst = reinterpret_cast<uint32_t*>(v_cache + (slot * hkv + hh - hkv) * D + l16 * E);
 #pragma unroll
-          for (int i = 0; i < W; ++i) dst[i] = x[g][i];
-        }
-        continue;
+        for (int i = 0; i < W; ++i) dst[i] = x[g][i];
       }
+      continue;
     }
     const uint32_t* wp = reinterpret_cast<const uint32_t*>((is_q ? qw : kw) + l16 * E);
     float v[E], wv[E];
@@ -186,10 +233,10 @@ __global__ __launch_bounds__(kQkWaves * 64) void qk_norm_rope_kernel(
       y[i] = pack_bf16x2(o[0], o[1]);
     }
     if (head >= heads || (!is_q && !slot_ok)) continue;
-    const bool is_v = APPEND && !is_q && hh >= hkv;
+    const bool is_v = !is_q && hh >= hkv;
     bf16* dst = is_q   ? q_out + (t * hq + hh) * D
-                : is_v ? v_out + (slot * hkv + hh - hkv) * D
-                       : k_out + ((APPEND ? slot : t) * hkv + hh) * D;
+                : is_v ? v_cache + (slot * hkv + hh - hkv) * D
+                       : k_cache + (slot * hkv + hh) * D;
 #pragma unroll
     for (int i = 0; i < W; ++i)
       reinterpret_cast<uint32_t*>(dst + l16 * E)[i] = is_v ? x[g][i] : y[i];
@@ -235,38 +282,66 @@ bool rmsnorm_supported(int hidden) {
 hipError_t qk_norm_rope(const void* qkv, int64_t stride, int64_t tokens, int hq, int hkv, int D,
                         const void* qw, const void* kw, const float* cos_t, const float* sin_t,
                         int64_t table_rows, const int32_t* positions, void* q_out, void* k_out,
-                        float eps, void* v_out, int64_t num_slots, const int32_t* out_loc,
-                        hipStream_t stream) {
+                        float eps, hipStream_t stream) {
   if (tokens == 0) return hipSuccess;
-  const bool append = v_out != nullptr;
-  const int heads = hq + (append ? 2 : 1) * hkv;
-  // Several groups per wavefront once one each is 16 wavefronts per compute unit.
-  const bool many = tokens * ((heads + 3) / 4) >= 4096;
-  const int64_t sets = many ? (heads + 7) / 8 : (heads + 3) / 4;
-  const dim3 grid((unsigned)((tokens * sets + kQkWaves - 1) / kQkWaves));
-#define AIOS_QKR(DD, AP, GPW)                                                                 \
-  hipLaunchKernelGGL((qk_norm_rope_kernel<DD, AP, GPW>), grid, dim3(kQkWaves * 64), 0, stream, \
-                     static_cast<const bf16*>(qkv), stride, tokens, hq, hkv,                  \
+  const dim3 grid((unsigned)tokens, (unsigned)((hq + hkv + 3) / 4));
+#define AIOS_QKR(DD)                                                                          \
+  hipLaunchKernelGGL(qk_norm_rope_kernel<DD>, grid, dim3(64), 0, stream,                      \
+                     static_cast<const bf16*>(qkv), stride, hq, hkv,                          \
                      static_cast<const bf16*>(qw), static_cast<const bf16*>(kw), cos_t, sin_t, \
-                     table_rows, positions, static_cast<bf16*>(q_out),                        \
-                     static_cast<bf16*>(k_out), eps, static_cast<bf16*>(v_out), num_slots, out_loc)
-#define AIOS_QKRD(DD)                                                      \
-  do {                                                                     \
-    if (append) {                                                          \
-      if (many) AIOS_QKR(DD, true, 2); else AIOS_QKR(DD, true, 1);         \
-    } else {                                                               \
-      if (many) AIOS_QKR(DD, false, 2); else AIOS_QKR(DD, false, 1);       \
-    }                                                                      \
-  } while (0)
+                     table_rows, positions, static_cast<bf16*>(q_out), static_cast<bf16*>(k_out), eps)
   switch (D) {
-    case 64: AIOS_QKRD(64); break;
-    case 96: AIOS_QKRD(96); break;
-    case 128: AIOS_QKRD(128); break;
+    case 64: AIOS_QKR(64); break;
+    case 96: AIOS_QKR(96); break;
+    case 128: AIOS_QKR(128); break;
     default: return hipErrorInvalidValue;
   }
-#undef AIOS_QKRD
 #undef AIOS_QKR
   return hipGetLastError();
+}
+
+template <int D>
+static hipError_t launch_rope_append(const void* qkv, int64_t stride, int64_t tokens, int hq, int hkv,
+                                     const void* qw, const void* kw, const float* cos_t,
+                                     const float* sin_t, int64_t table_rows, const int32_t* positions,
+                                     void* q_out, void* k_cache, void* v_cache, int64_t num_slots,
+                                     const int32_t* out_loc, float eps, hipStream_t stream) {
+  const int heads = hq + 2 * hkv;
+  auto launch = [&](auto kernel, int sets) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)tokens, (unsigned)sets), dim3(64), 0, stream,
+                       static_cast<const bf16*>(qkv), stride, hq, hkv, static_cast<const bf16*>(qw),
+                       static_cast<const bf16*>(kw), cos_t, sin_t, table_rows, positions,
+                       static_cast<bf16*>(q_out), static_cast<bf16*>(k_cache),
+                       static_cast<bf16*>(v_cache), num_slots, out_loc, eps);
+    return hipGetLastError();
+  };
+  // Two groups per wavefront once one each is 16 wavefronts per compute unit.
+  return tokens * ((heads + 3) / 4) >= 4096
+             ? launch(qk_norm_rope_append_kernel<D, 2>, (heads + 7) / 8)
+             : launch(qk_norm_rope_append_kernel<D, 1>, (heads + 3) / 4);
+}
+
+hipError_t qk_norm_rope_append(const void* qkv, int64_t stride, int64_t tokens, int hq, int hkv, int D,
+                               const void* qw, const void* kw, const float* cos_t,
+                               const float* sin_t, int64_t table_rows, const int32_t* positions,
+                               void* q_out, void* k_cache, void* v_cache, int64_t num_slots,
+                               const int32_t* out_loc, float eps, hipStream_t stream) {
+  if (tokens == 0) return hipSuccess;
+  switch (D) {
+    case 64:
+      return launch_rope_append<64>(qkv, stride, tokens, hq, hkv, qw, kw, cos_t, sin_t, table_rows,
+                                    positions, q_out, k_cache, v_cache, num_slots, out_loc, eps,
+                                    stream);
+    case 96:
+      return launch_rope_append<96>(qkv, stride, tokens, hq, hkv, qw, kw, cos_t, sin_t, table_rows,
+                                    positions, q_out, k_cache, v_cache, num_slots, out_loc, eps,
+                                    stream);
+    case 128:
+      return launch_rope_append<128>(qkv, stride, tokens, hq, hkv, qw, kw, cos_t, sin_t, table_rows,
+                                     positions, q_out, k_cache, v_cache, num_slots, out_loc, eps,
+                                     stream);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t silu_mul(const void* x, int64_t x_stride, int64_t rows, int inter, void* out,
