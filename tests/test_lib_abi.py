@@ -145,6 +145,16 @@ def test_plan_prefill_split_of_batches(reqs, q, kv, hq, hkv, d, split):
     assert rc == 0 and (p.num_parts > 1) == split
 
 
+@pytest.mark.parametrize("rows,n,k,split", [
+    # one row tile: K split over workgroups only where that is the faster form
+    (8, 1024, 2560, False), (16, 1024, 2560, True), (1, 64, 1280, False), (4, 2560, 4096, False),
+    (16, 2560, 4096, True), (8, 4096, 4096, False), (1, 2560, 9728, True), (8, 1024, 2048, False),
+    (24, 1024, 3072, True), (24, 6144, 2560, False), (17, 512, 128, False),
+])
+def test_projections_that_split_k(rows, n, k, split):
+    assert (_lib.lib().aios_linear_rows_workspace(rows, n, k) > 0) == split
+
+
 def test_plan_rejects_bad_batches():
     lib = _lib.lib()
     rc, _ = _plan(_lib.PHASE_DECODE, [0, 2], [0, 5])  # two query tokens in decode
