@@ -112,10 +112,15 @@ class HipOps:
         n = weight.shape[0] // 2 if silu else weight.shape[0]
         rows_ok = self._rows_ok(h, weight, k) and n % 16 == 0
         # One 16-row tile whose normalised fragments fit the registers (K / 128
-        # of them, at most 8) takes the norm in the projection's launch; more
-        # rows pay less for it as a launch of its own than for forming it in
-        # every workgroup (24 x 768 x 1280: 6.7 us against 9 in two tiles).
-        if (rows_ok and rows <= 16 and k <= 1024
+        # of them, at most 8) takes the norm in the projection's launch.  More
+        # tiles do while forming it in every workgroup costs less than a launch
+        # (24 x 128 x 256 3.1 us against 4.8, 32 x 512 x 1024 5.0 against 5.7
+        # without a residual, 5.8 against 5.3 with one; 24 x 768 x 1280, in two
+        # launches, 9 against 6.7).
+        frags = k // 128 * -(-rows // 16)
+        few = rows <= 16 or (frags + 2 * (residual is not None) + 2 * silu <= 8
+                             and frags * n <= 32768)
+        if (rows_ok and few and frags <= 8
                 and (residual is None
                      or (residual.stride(1) == 1 and residual.stride(0) % 8 == 0))):
             _check_gpu(h, weight, norm_weight, *(() if residual is None else (residual,)))

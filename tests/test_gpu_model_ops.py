@@ -5,6 +5,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from aios_amd import _lib
 from aios_amd.layers import HipOps
 from aios_amd.qwen3 import RotaryEmbedding
 from tests.util import TorchOps
@@ -137,8 +138,8 @@ def test_linear_rows_strided_input_and_fallback():
 def test_add_rmsnorm_linear(rows, k, n, with_residual):
     """RMSNorm (with the residual add) folded into the projection: the same
     normalised operand as the separate kernels, the residual sum bit-exact;
-    more rows than one launch holds (17, 24 at K 768 / 1024; 40 at K 512)
-    run as row chunks."""
+    more rows or a longer K than that pays for (17, 24 at K 768 / 1024, 40 at
+    K 512, K 2048) run as norm, then projection."""
     h = _bf16((rows, k), rows + k, 2.0)
     r = _bf16((rows, k), rows + k + 1, 3.0) if with_residual else None
     nw = _bf16((k,), 9).abs() + 0.5
@@ -154,6 +155,43 @@ def test_add_rmsnorm_linear(rows, k, n, with_residual):
     y_ref = x_ref.float() @ w.float().T
     err = (y.float() - y_ref).abs()
     assert bool((err <= 2.0 ** -7 * y_ref.abs() + 2e-3 * y_ref.abs().max()).all()), err.max().item()
+
+
+@pytest.mark.parametrize("rows,k,n", [(17, 128, 256), (32, 512, 1024), (32, 384, 48), (33, 256, 512),
+                                      (48, 128, 16), (64, 256, 272), (64, 128, 8208)])
+@pytest.mark.parametrize("silu", [False, True])
+@pytest.mark.parametrize("with_residual", [True, False])
+@pytest.mark.parametrize("folded", [True, False])
+def test_norm_of_several_row_tiles(rows, k, n, silu, with_residual, folded):
+    """The norm in front of two to four 16-row tiles, in the projection's launch
+    (called directly: add_rmsnorm_linear takes it for some of these sizes) and
+    as add_rmsnorm_linear runs it."""
+    h = _bf16((rows, k), rows + k, 2.0)
+    r = _bf16((rows, k), rows + k + 1, 3.0) if with_residual else None
+    nw = _bf16((k,), 9).abs() + 0.5
+    w = _bf16((2 * n if silu else n, k), n, 0.05)
+    if folded:
+        y, new_r = torch.empty(rows, n, dtype=h.dtype, device=DEV), torch.empty_like(h)
+        _lib.check(_lib.lib().aios_linear_rows_ex(
+            h.data_ptr(), k, w.data_ptr(), k, y.data_ptr(), n, rows, n, k,
+            _lib.PROLOGUE_ADD_RMSNORM, r.data_ptr() if with_residual else None,
+            k if with_residual else 0, nw.data_ptr(), 1e-6,
+            new_r.data_ptr() if with_residual else None, k if with_residual else 0,
+            _lib.EPILOGUE_SILU_MUL if silu else _lib.EPILOGUE_NONE, 0), "aios_linear_rows_ex")
+        torch.cuda.synchronize()
+    else:
+        y, new_r = HipOps().add_rmsnorm_linear(h, r, nw, 1e-6, w, silu=silu)
+    ref = TorchOps()
+    x_ref = ref.rmsnorm(h, nw, 1e-6)
+    if with_residual:
+        x_ref, r_ref = ref.fused_add_rmsnorm(h.clone(), r.clone(), nw, 1e-6)
+        assert torch.equal(new_r, r_ref)
+    y_ref = x_ref.float() @ w.float().T
+    if silu:
+        y_ref = ref.silu_and_mul(y_ref.to(torch.bfloat16)).float()
+    err = (y.float() - y_ref).abs()
+    tol = 2.0 ** -6 if silu else 2.0 ** -7
+    assert bool((err <= tol * y_ref.abs() + 4e-3 * y_ref.abs().max()).all()), err.max().item()
 
 
 @pytest.mark.parametrize("rows,k,inter", [(8, 768, 2048), (3, 512, 256), (33, 256, 512),

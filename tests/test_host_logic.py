@@ -280,6 +280,27 @@ def test_one_host_operand_is_refused(on_host, monkeypatch):
     assert lib.calls == []
 
 
+@pytest.mark.parametrize("rows,k,n,residual,silu,folded", [
+    (16, 1024, 512, True, True, True), (17, 1024, 512, False, False, False),
+    (24, 128, 256, True, True, True), (64, 128, 256, True, True, True),
+    (32, 256, 512, True, True, True), (33, 256, 512, True, True, False),
+    (33, 256, 512, False, True, True), (32, 512, 1024, False, False, True),
+    (32, 512, 1024, True, False, False), (32, 512, 8192, False, False, False),
+    (8, 2048, 512, False, False, False),
+])
+def test_norm_folded_where_it_pays(rows, k, n, residual, silu, folded, monkeypatch):
+    """More than one 16-row tile takes the norm in the projection's launch only
+    while that measured faster than a launch of its own."""
+    lib = _NoLaunch()
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    monkeypatch.setattr(_lib, "raw_stream", lambda device: 0)
+    t = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16).as_subclass(_GpuTensor)
+    HipOps().add_rmsnorm_linear(t(rows, k), t(rows, k) if residual else None, t(k), 1e-6,
+                                t(n * (1 + silu), k), silu=silu)
+    assert (lib.calls == ["aios_linear_rows_ex"]) == folded
+    assert folded or lib.calls[0] in ("aios_rmsnorm", "aios_add_rmsnorm")
+
+
 @pytest.mark.parametrize("kind", ["decode", "prefill"])
 @pytest.mark.parametrize("enabled", [True, False])
 @pytest.mark.parametrize("fails", [False, True])
