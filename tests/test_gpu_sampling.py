@@ -273,7 +273,7 @@ def test_sample_split_rows(dtype, vocab):
 def test_sample_split_rows_tied_beyond_the_candidate_buffer(dtype):
     """Four distinct values over 151,936 ids: every segment's candidates are the
     lowest of its ties, and the row's overflow the merge's buffer too, so the
-    cut among them is found by bisection on (value, id)."""
+    cut among them is found from counts over ranges of (value, id)."""
     rows, vocab = 4, 151936
     g = torch.Generator(device="cuda").manual_seed(12)
     x = (torch.randint(0, 4, (rows, vocab), generator=g, device="cuda").to(torch.float32) * 0.5).to(dtype)
@@ -285,3 +285,17 @@ def test_sample_split_rows_tied_beyond_the_candidate_buffer(dtype):
                    SamplingParams(temperature=0.0)):
         _check_rows(x, params, u)
         _check_rows(x, params, u, forbidden=(3,), by_row=by_row)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [20000, 65544, 151936])
+@pytest.mark.parametrize("scale", [1e-6, 1e-3, 0.05, 2.0])
+def test_sample_split_rows_close_beyond_the_candidate_buffer(dtype, vocab, scale):
+    """Values so close (or so few in bf16) that more than the merge's buffer lie
+    within its first bound: one to several passes narrow the cut."""
+    rows = 4
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    x = (1.0 + torch.randn(rows, vocab, generator=g, device="cuda") * scale).to(dtype)
+    u = stateless_uniforms([70 + r for r in range(rows)], 1, torch.device("cuda"))[:, 0]
+    for k in (1, 700, 1024):
+        _check_rows(x, SamplingParams(temperature=1.0, top_k=k, top_p=1.0), u, forbidden=(3, vocab - 1))
