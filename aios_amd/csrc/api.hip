@@ -174,15 +174,13 @@ void plan_prefill_parts(aios_attn_plan_t* p, const int32_t* cu_q, const int32_t*
     return;
   const int64_t parts = (int64_t)p->batch_size * p->num_q_tiles * hkv * n;
   const int64_t o_bytes = align_up(parts * rows * p->head_dim * 4, 256);
-  const int64_t bytes = n > 1 ? o_bytes + align_up(parts * rows * 8, 256) : 0;
+  const int64_t bytes = o_bytes + align_up(parts * rows * 8, 256);
   if (bytes > ws_bytes || parts > 0x3fffffff) return;
   p->prefix_chunk_len = part_sub * 32;
-  p->num_parts = n;
-  if (n > 1) {
-    p->ws_parts_o = 0;
-    p->ws_parts_lse = o_bytes;
-    p->ws_bytes = bytes;
-  }
+  p->num_parts = n;  // (at least 2: every line above leaves shorter ranges whole)
+  p->ws_parts_o = 0;
+  p->ws_parts_lse = o_bytes;
+  p->ws_bytes = bytes;
 }
 
 }  // namespace
