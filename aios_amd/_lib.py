@@ -102,14 +102,14 @@ class AttnPlan(ctypes.Structure):
         return {name: getattr(self, name) for name, _ in self._fields_}
 
 
-def raw_stream(device) -> int:
-    """The current HIP stream handle of a torch GPU device (the handle alone:
+def raw_stream(t: torch.Tensor) -> int:
+    """The current HIP stream handle of a GPU tensor's device (the handle alone:
     torch.cuda.current_stream builds a Stream object, 2 us of each launch).
-    Another device has none: its tensors' addresses must not reach a kernel."""
-    if device.type != "cuda":
-        raise ValueError(f"expected a GPU device, got {device}")
-    index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    Other tensors have none: their addresses must not reach a kernel."""
+    index = t.get_device()
+    if index < 0:
+        raise ValueError(f"expected a GPU tensor, got one on {t.device}")
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 _lock = threading.Lock()

@@ -17,7 +17,7 @@ from aios_amd import _lib
 
 
 def _stream(t: torch.Tensor) -> int:
-    return _lib.raw_stream(t.device)
+    return _lib.raw_stream(t)
 
 
 def _check_bank(bank: torch.Tensor) -> tuple[int, int, int]:

@@ -39,7 +39,7 @@ def store_cache(
     if indices.dtype != torch.int32:
         indices = indices.to(torch.int32)
     indices = indices.contiguous()
-    stream = _lib.raw_stream(k_cache.device)
+    stream = _lib.raw_stream(k_cache)
     _lib.check(
         _lib.lib().aios_kv_append(
             k_cache.data_ptr(),

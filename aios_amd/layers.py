@@ -15,7 +15,7 @@ from aios_amd import _lib
 
 
 def _stream(t: torch.Tensor) -> int:
-    return _lib.raw_stream(t.device)
+    return _lib.raw_stream(t)
 
 
 def _check_gpu(*tensors: torch.Tensor) -> None:
@@ -117,10 +117,10 @@ class HipOps:
         # (24 x 128 x 256 3.1 us against 4.8, 32 x 512 x 1024 5.0 against 5.7
         # without a residual, 5.8 against 5.3 with one; 24 x 768 x 1280, in two
         # launches, 9 against 6.7).
-        frags = k // 128 * -(-rows // 16)
-        few = rows <= 16 or (frags + 2 * (residual is not None) + 2 * silu <= 8
-                             and frags * n <= 32768)
-        if (rows_ok and few and frags <= 8
+        frags = k // 128 * -(-rows // 16) if rows_ok else 9
+        if (frags <= 8
+                and (rows <= 16 or (frags + 2 * (residual is not None) + 2 * silu <= 8
+                                    and frags * n <= 32768))
                 and (residual is None
                      or (residual.stride(1) == 1 and residual.stride(0) % 8 == 0))):
             _check_gpu(h, weight, norm_weight, *(() if residual is None else (residual,)))

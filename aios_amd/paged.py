@@ -13,8 +13,8 @@ from aios_amd import _lib
 DEFAULT_WORKSPACE = 128 * 1024 * 1024
 
 
-def _stream(device: torch.device) -> int:
-    return _lib.raw_stream(device)
+def _stream(t: torch.Tensor) -> int:
+    return _lib.raw_stream(t)
 
 
 def _host_i32(x) -> torch.Tensor:
@@ -89,7 +89,7 @@ def decode(p: _lib.AttnPlan, q: torch.Tensor, k_cache: torch.Tensor, v_cache: to
             p, q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
             k_cache.shape[0], indices.data_ptr(), cu_k.data_ptr(), out.data_ptr(),
             workspace.data_ptr() if workspace is not None else None,
-            workspace.numel() if workspace is not None else 0, scale, _stream(q.device)),
+            workspace.numel() if workspace is not None else 0, scale, _stream(q)),
         "aios_attn_decode",
     )
     return out
@@ -117,7 +117,7 @@ def decode_noalloc(p: _lib.AttnPlan, q: torch.Tensor, k_cache: torch.Tensor,
         _lib.lib().aios_attn_decode_noalloc(
             p, q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
             k_cache.shape[0], indices.data_ptr(), cu_k.data_ptr(), out.data_ptr(), scale,
-            _stream(q.device)),
+            _stream(q)),
         "aios_attn_decode_noalloc",
     )
     return out
@@ -164,7 +164,7 @@ def append_decode(p: _lib.AttnPlan, q: torch.Tensor, k: torch.Tensor, v: torch.T
             out_loc.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), k_cache.shape[0],
             indices.data_ptr(), cu_k.data_ptr(), out.data_ptr(),
             workspace.data_ptr() if workspace is not None else None,
-            workspace.numel() if workspace is not None else 0, scale, _stream(q.device)),
+            workspace.numel() if workspace is not None else 0, scale, _stream(q)),
         "aios_attn_append_decode",
     )
     return out
@@ -212,7 +212,7 @@ def append_decode_rope(p: _lib.AttnPlan, q: torch.Tensor, k: torch.Tensor, v: to
             indices.data_ptr(), cu_k.data_ptr(), q_norm.data_ptr(), k_norm.data_ptr(),
             cos.data_ptr(), sin.data_ptr(), cos.shape[0], positions.data_ptr(), float(eps),
             out.data_ptr(), workspace.data_ptr() if workspace is not None else None,
-            workspace.numel() if workspace is not None else 0, scale, _stream(q.device)),
+            workspace.numel() if workspace is not None else 0, scale, _stream(q)),
         "aios_attn_append_decode_rope",
     )
     return out
@@ -243,7 +243,7 @@ def prefill(p: _lib.AttnPlan, q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
         _lib.lib().aios_attn_prefill_ws(
             p, q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
             k_cache.shape[0], indices.data_ptr(), cu_q.data_ptr(), cu_k.data_ptr(), out.data_ptr(),
-            ws.data_ptr() if ws is not None else None, p.ws_bytes, scale, _stream(q.device)),
+            ws.data_ptr() if ws is not None else None, p.ws_bytes, scale, _stream(q)),
         "aios_attn_prefill_ws",
     )
     return out
@@ -260,7 +260,7 @@ def build_indices(page_table: torch.Tensor, row_ids: torch.Tensor, cu_k: torch.T
     _lib.check(
         _lib.lib().aios_build_indices(page_table.data_ptr(), page_table.stride(0),
                                       row_ids.data_ptr(), cu_k.data_ptr(), row_ids.numel(),
-                                      total_kv, out.data_ptr(), _stream(page_table.device)),
+                                      total_kv, out.data_ptr(), _stream(page_table)),
         "aios_build_indices",
     )
     return out
@@ -288,7 +288,7 @@ def greedy_select(logits: torch.Tensor,
     _lib.check(
         _lib.lib().aios_greedy_select(logits.data_ptr(), logits.stride(0), rows, vocab,
                                       logits.element_size(), tok.data_ptr(), lp.data_ptr(),
-                                      _stream(logits.device)),
+                                      _stream(logits)),
         "aios_greedy_select",
     )
     return tok, lp
@@ -328,7 +328,7 @@ def bind_decode(p: _lib.AttnPlan, q: torch.Tensor, k_cache: torch.Tensor, v_cach
     if p.ws_bytes and (workspace is None or workspace.numel() < p.ws_bytes):
         raise RuntimeError(f"decode needs a workspace of {p.ws_bytes} bytes")
     scale = p.head_dim ** -0.5 if sm_scale is None else sm_scale
-    s = stream.cuda_stream if stream is not None else _stream(q.device)
+    s = stream.cuda_stream if stream is not None else _stream(q)
     args = (ctypes.byref(p), q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
             k_cache.shape[0], indices.data_ptr(), cu_k.data_ptr(), out.data_ptr(),
             workspace.data_ptr() if workspace is not None else None,
@@ -356,7 +356,7 @@ def bind_append_decode(p: _lib.AttnPlan, q: torch.Tensor, k: torch.Tensor, v: to
     if p.ws_bytes and (workspace is None or workspace.numel() < p.ws_bytes):
         raise RuntimeError(f"decode needs a workspace of {p.ws_bytes} bytes")
     scale = p.head_dim ** -0.5 if sm_scale is None else sm_scale
-    s = stream.cuda_stream if stream is not None else _stream(q.device)
+    s = stream.cuda_stream if stream is not None else _stream(q)
     args = (ctypes.byref(p), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(),
             v.stride(0), out_loc.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
             k_cache.shape[0], indices.data_ptr(), cu_k.data_ptr(), out.data_ptr(),
@@ -376,7 +376,7 @@ def bind_kv_append(k_cache: torch.Tensor, v_cache: torch.Tensor, out_loc: torch.
         raise ValueError("out_loc must be a contiguous int32 tensor with one entry per token")
     if not all(t.is_cuda for t in (k_cache, v_cache, out_loc, k, v)):
         raise ValueError("the KV append takes GPU tensors")
-    s = stream.cuda_stream if stream is not None else _stream(k.device)
+    s = stream.cuda_stream if stream is not None else _stream(k)
     width = k_cache.shape[1] * k_cache.shape[2]
     args = (k_cache.data_ptr(), v_cache.data_ptr(), k_cache.shape[0], k_cache.stride(0),
             out_loc.data_ptr(), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), k.shape[0],

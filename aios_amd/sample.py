@@ -29,7 +29,7 @@ _NO_STEP_LIMIT = 2**31 - 1
 
 
 def _stream(t: torch.Tensor) -> int:
-    return _lib.raw_stream(t.device)
+    return _lib.raw_stream(t)
 
 
 def stateless_uniforms(candidate_seeds: Sequence[int] | torch.Tensor, steps: int,

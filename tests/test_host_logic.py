@@ -224,9 +224,8 @@ def _host_calls():
         "qk_norm_rope_append": append,
         "build_indices": lambda: paged.build_indices(i32(2, 8), i32(2), i32(3), 4),
         "bind_kv_append": lambda: paged.bind_kv_append(cache, cache, i32(3), kv, kv)(),
-        "raw_stream": lambda: _lib.raw_stream(torch.device("cpu")),
-        "raw_stream_indexed": lambda: _lib.raw_stream(torch.device("cpu", 0)),
-        "raw_stream_meta": lambda: _lib.raw_stream(torch.device("meta")),
+        "raw_stream": lambda: _lib.raw_stream(torch.zeros(1)),
+        "raw_stream_meta": lambda: _lib.raw_stream(torch.zeros(1, device="meta")),
     }
 
 
@@ -255,7 +254,7 @@ def test_one_host_operand_is_refused(on_host, monkeypatch):
     """Each operand of the calls above is checked for itself."""
     lib = _NoLaunch()
     monkeypatch.setattr(_lib, "lib", lambda: lib)
-    monkeypatch.setattr(_lib, "raw_stream", lambda device: 0)
+    monkeypatch.setattr(_lib, "raw_stream", lambda t: 0)
 
     def t(name, *shape, dtype=torch.bfloat16):
         x = torch.zeros(shape, dtype=dtype)
@@ -293,7 +292,7 @@ def test_norm_folded_where_it_pays(rows, k, n, residual, silu, folded, monkeypat
     while that measured faster than a launch of its own."""
     lib = _NoLaunch()
     monkeypatch.setattr(_lib, "lib", lambda: lib)
-    monkeypatch.setattr(_lib, "raw_stream", lambda device: 0)
+    monkeypatch.setattr(_lib, "raw_stream", lambda t: 0)
     t = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16).as_subclass(_GpuTensor)
     HipOps().add_rmsnorm_linear(t(rows, k), t(rows, k) if residual else None, t(k), 1e-6,
                                 t(n * (1 + silu), k), silu=silu)
