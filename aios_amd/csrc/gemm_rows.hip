@@ -1,6 +1,7 @@
 // Few-row projections y[M, N] = x[M, K] W[N, K]^T that stream their weights
-// past resident rows: 17 to 64 rows, or a K outside the fixed-K instances of
-// gemm_skinny.hip (bf16 in, fp32 accumulate, bf16 out).
+// past resident rows: 17 to 64 rows, and the K of fewer rows for which that
+// measured faster than gemm_skinny.hip (rows_form in api.hip; bf16 in, fp32
+// accumulate, bf16 out).
 //
 // What bounds a few-row projection is how fast a compute unit takes in
 // operands: about 25-30 bytes per nanosecond (measured, HBM and L2 alike), and
