@@ -150,24 +150,25 @@ __global__ __launch_bounds__(64) void qk_norm_rope_kernel(
 // entries are the same for every head of its token: with many tokens a
 // wavefront takes GPW groups of four heads and reads them once (the fp32 tables
 // are four times a head's bytes), with few tokens one group each, for the
-// parallelism.  Per launch in a graph, a 2-D grid against workgroups of four
-// wavefronts that divided their index by the head sets: 6 tokens of 32q/8kv x
-// 128 2.58 -> 2.37 us, 2,048 of 16q/8kv x 128 10.0 -> 9.4 (traced, with the
-// two launches it stands for 5.0 + 4.5 -> 4.1 and 8.2 + 5.0 -> 10.4).
-template <int D, int GPW>
-__global__ __launch_bounds__(64) void qk_norm_rope_append_kernel(
+// parallelism.  Against workgroups of four wavefronts that divided their index
+// by the head sets: 6 tokens of 32q/8kv x 128 2.58 -> 2.37 us per launch in a
+// graph, 2,048 of 16q/8kv x 128 10.8 -> 10.4 traced in a model's prefill (the
+// two launches it stands for: 5.0 + 4.5 and 8.2 + 5.0 traced).
+template <int D, int GPW, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void qk_norm_rope_append_kernel(
     const bf16* __restrict__ qkv, int64_t stride, int hq, int hkv, const bf16* __restrict__ qw,
     const bf16* __restrict__ kw, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, int64_t table_rows, const int32_t* __restrict__ positions,
     bf16* __restrict__ q_out, bf16* __restrict__ k_cache, bf16* __restrict__ v_cache,
-    int64_t num_slots, const int32_t* __restrict__ out_loc, float eps) {
+    int64_t num_slots, const int32_t* __restrict__ out_loc, float eps, int64_t tokens) {
   constexpr int E = D / 16;
   constexpr int W = E / 2;  // 32-bit words per lane
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   const int l16 = lane & 15;
   const int heads = hq + 2 * hkv;
   const int head0 = blockIdx.y * 4 * GPW + (lane >> 4);
-  const int64_t t = blockIdx.x;
+  const int64_t t = (int64_t)blockIdx.x * WAVES + (threadIdx.x >> 6);
+  if (t >= tokens) return;
   // Positions outside the table are clamped (never read out of bounds).
   const int64_t pos = min(max((int64_t)positions[t], (int64_t)0), table_rows - 1);
   const int64_t slot = out_loc[t];
@@ -312,18 +313,22 @@ static hipError_t launch_rope_append(const void* qkv, int64_t stride, int64_t to
                                      void* q_out, void* k_cache, void* v_cache, int64_t num_slots,
                                      const int32_t* out_loc, float eps, hipStream_t stream) {
   const int heads = hq + 2 * hkv;
-  auto launch = [&](auto kernel, int sets) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)tokens, (unsigned)sets), dim3(64), 0, stream,
+  auto launch = [&](auto kernel, int sets, int waves) {
+    const dim3 grid((unsigned)((tokens + waves - 1) / waves), (unsigned)sets);
+    hipLaunchKernelGGL(kernel, grid, dim3(waves * 64), 0, stream,
                        static_cast<const bf16*>(qkv), stride, hq, hkv, static_cast<const bf16*>(qw),
                        static_cast<const bf16*>(kw), cos_t, sin_t, table_rows, positions,
                        static_cast<bf16*>(q_out), static_cast<bf16*>(k_cache),
-                       static_cast<bf16*>(v_cache), num_slots, out_loc, eps);
+                       static_cast<bf16*>(v_cache), num_slots, out_loc, eps, tokens);
     return hipGetLastError();
   };
-  // Two groups per wavefront once one each is 16 wavefronts per compute unit.
-  return tokens * ((heads + 3) / 4) >= 4096
-             ? launch(qk_norm_rope_append_kernel<D, 2>, (heads + 7) / 8)
-             : launch(qk_norm_rope_append_kernel<D, 1>, (heads + 3) / 4);
+  // Two groups per wavefront once one each is 16 wavefronts per compute unit;
+  // two tokens per workgroup from 6 on (256 tokens of 16q/8kv x 128 3.14 us
+  // against 2.95, 100 of 32q/8kv 2.66 against 2.82).
+  const int64_t units = tokens * ((heads + 3) / 4);
+  if (units >= 4096) return launch(qk_norm_rope_append_kernel<D, 2, 2>, (heads + 7) / 8, 2);
+  if (units >= 1536) return launch(qk_norm_rope_append_kernel<D, 1, 2>, (heads + 3) / 4, 2);
+  return launch(qk_norm_rope_append_kernel<D, 1, 1>, (heads + 3) / 4, 1);
 }
 
 hipError_t qk_norm_rope_append(const void* qkv, int64_t stride, int64_t tokens, int hq, int hkv, int D,

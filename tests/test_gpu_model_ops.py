@@ -67,7 +67,11 @@ def test_qk_norm_rope(hq, hkv, d):
 
 
 @pytest.mark.parametrize("hq,hkv,d,t", [(8, 2, 96, 1), (12, 4, 64, 19), (16, 8, 128, 5),
-                                        (8, 8, 64, 3), (32, 8, 128, 130)])
+                                        (8, 8, 64, 3), (32, 8, 128, 130),
+                                        # two tokens a workgroup, then two head
+                                        # groups a wavefront (one past the line, odd)
+                                        (8, 2, 96, 513), (16, 8, 128, 513), (12, 4, 64, 821),
+                                        (8, 2, 96, 1367)])
 def test_qk_norm_rope_append_is_the_two_calls(hq, hkv, d, t):
     """The same bits as qk_norm_rope and store_cache, rows of other slots left
     alone, slots outside the pool skipped; qkv rows with a gap between them."""
