@@ -12,6 +12,7 @@ from __future__ import annotations
 import torch
 
 from aios_amd import _lib
+from aios_amd.core import runs_as_built
 
 
 def _stream(t: torch.Tensor) -> int:
@@ -35,13 +36,21 @@ def _plain_rows(t: torch.Tensor) -> bool:
             and t.data_ptr() % 16 == 0)
 
 
+def _plain_copy(t: torch.Tensor, name: str) -> torch.Tensor:
+    """t, or a copy where its rows cannot be read in place."""
+    if _plain_rows(t):
+        if t.dtype == torch.bfloat16 and t.is_cuda:
+            return t
+    else:
+        t = t.clone()
+    _check_rows(t, name)
+    return t
+
+
 def _add_rmsnorm(h: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                  eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """(RMSNorm(h + residual) * weight, h + residual), the inputs left unchanged."""
-    h = h if _plain_rows(h) else h.clone()
-    residual = residual if _plain_rows(residual) else residual.clone()
-    _check_rows(h, "x")
-    _check_rows(residual, "residual")
+    h, residual = _plain_copy(h, "x"), _plain_copy(residual, "residual")
     if h.shape != residual.shape:
         raise ValueError("x and residual must have the same shape")
     out, total = torch.empty_like(h), torch.empty_like(residual)
@@ -138,9 +147,11 @@ class HipOps:
             return y, total
         if residual is None:
             x, residual = self.rmsnorm(h, norm_weight, eps), h
-        else:
+        elif runs_as_built(self, _FUSED_NORM):
             x, residual = _add_rmsnorm(h, residual, norm_weight, eps)
-        if silu and rows_ok and k <= 2560:
+        else:  # (a caller's own in-place norm, the inputs left unchanged)
+            x, residual = self.fused_add_rmsnorm(h.clone(), residual.clone(), norm_weight, eps)
+        if silu and rows_ok and k <= 2560 and runs_as_built(self, _LINEAR_SILU):
             return _linear_rows(x, weight, n, silu=True), residual
         y = self.linear(x, weight)
         return (self.silu_and_mul(y) if silu else y), residual
@@ -248,3 +259,8 @@ class HipOps:
                                             out.data_ptr(), out.stride(0), _stream(x)),
                    "aios_silu_mul")
         return out
+
+
+# The ops that add_rmsnorm_linear's separate launches stand for, as built here.
+_FUSED_NORM = (("fused_add_rmsnorm", HipOps.fused_add_rmsnorm),)
+_LINEAR_SILU = (("linear", HipOps.linear), ("silu_and_mul", HipOps.silu_and_mul))

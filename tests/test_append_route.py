@@ -187,3 +187,35 @@ def test_own_ops_and_backends_see_every_prefill(kind):
         assert log == ["layer_kv", "append", "appended"]
     else:
         assert "append" not in log and log[-1] == "forward" and "rope" in log
+
+
+class _NoLaunch:
+    def __getattr__(self, name):
+        return lambda *args: 0
+
+
+@pytest.mark.parametrize("how", ["subclass", "attribute"])
+@pytest.mark.parametrize("name,rows,k,silu", [("fused_add_rmsnorm", 8, 2560, False),
+                                              ("linear", 8, 2560, True),
+                                              ("silu_and_mul", 24, 1280, True)])
+def test_own_parts_of_the_norm_and_projection_are_called(how, name, rows, k, silu, monkeypatch):
+    """add_rmsnorm_linear outside the folded launch goes through the op set's own
+    residual-add norm, projection and activation."""
+    monkeypatch.setattr(_lib, "lib", lambda: _NoLaunch())
+    monkeypatch.setattr(_lib, "raw_stream", lambda t: 0)
+    empty, like = torch.empty, torch.empty_like
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: empty(*a, **k).as_subclass(_GpuTensor))
+    monkeypatch.setattr(torch, "empty_like", lambda x: like(x).as_subclass(_GpuTensor))
+    log = []
+
+    def own(*args):
+        log.append(name)
+        return getattr(HipOps, name)(*args)
+
+    if how == "subclass":
+        ops = type("Own", (HipOps,), {name: staticmethod(own)})()
+    else:
+        ops = _with(HipOps(), **{name: own})
+    t = lambda *shape: torch.zeros(shape, dtype=BF).as_subclass(_GpuTensor)
+    ops.add_rmsnorm_linear(t(rows, k), t(rows, k), t(k), 1e-6, t(64, k), silu=silu)
+    assert log == [name]
