@@ -81,20 +81,26 @@ int device_cus() {
 // gemm_skinny.hip keeps
 //  - up to one 16-column tile per unit, where streaming has no second tile to
 //    load ahead, a K to 1,792 (8 rows, 1024 x 1280 3.5 us against 3.9; 2560 x
-//    1280 4.0 against 4.1; with SiLU only its 8-column tiles, 2048 x 1280 6%);
+//    1280 4.0 against 4.1; with SiLU from 1,025 columns on, to 2,048, or to
+//    3,072 with K 1,280: 16 rows, 2560 x 1280 6.9 against 7.3);
 //  - its narrower tiles (at most one per two units) a K to 2,304, and to 2,688
-//    for up to 12 rows (8 rows, 1024 x 2560 4.9 against 5.6);
+//    for up to 12 rows (8 rows, 1024 x 2560 4.9 against 5.6) or where no
+//    workspace lets K be split (16 rows 5.9 against 6.5);
 //  - a K that has to be split, with its second launch, for few rows (1 row,
 //    2560 x 4096 7.8 against 8.5; 16 rows 11.0 against 9.8), and for close to
 //    one tile per unit (8 rows, 4096 x 4096 26% less).
-bool rows_form(int64_t rows, int64_t n, int64_t k, bool silu, int32_t cus) {
-  if (rows > 16) return true;
+// More rows with SiLU and a K to 384 stay there too: the streaming form has one
+// K step per wavefront and registers for three (24 rows, 6144 x 256 5.0 us
+// against 5.6).
+bool rows_form(int64_t rows, int64_t n, int64_t k, bool silu, bool workspace, int32_t cus) {
+  if (rows > 16) return !(silu && k <= 384);
   if (k <= 1024 || k == 2048 || k == 3072) return false;
   const int64_t tiles = n / 16;
-  if (silu) return 4 * tiles <= cus || 2 * tiles > cus || k > 1792;
-  if (tiles > cus) return rows > 2 || k < 3072 || k > 4096;
+  if (silu)
+    return 4 * tiles <= cus || !((2 * tiles <= cus && k <= 1792) || (4 * tiles <= 3 * cus && k <= 1280));
+  if (tiles > cus) return rows > 2 || (k > 1280 && (k < 3072 || k > 4096));
   if (k <= 1792 || (8 * tiles > 7 * cus && k <= 4608)) return false;
-  if (k <= 2688) return 2 * tiles > cus || (k > 2304 && rows > 12);
+  if (k <= 2688) return 2 * tiles > cus || (k > 2304 && rows > 12 && workspace);
   return k > 4608 || rows > 8 || n < (rows <= 4 && k <= 4096 ? 1024 : 2048);
 }
 
@@ -877,7 +883,7 @@ int aios_linear_rows_ex(const void* x, int64_t x_stride, const void* weight, int
 int64_t aios_linear_rows_workspace(int64_t rows, int64_t out_features, int64_t in_features) {
   aios::RowsPlan p;
   if (!aios::skinny_gemm_supported(rows, out_features, in_features) ||
-      !rows_form(rows, out_features, in_features, false, device_cus()) ||
+      !rows_form(rows, out_features, in_features, false, true, device_cus()) ||
       !aios::rows_gemm_plan(rows, out_features, in_features, false, true, device_cus(), &p))
     return 0;
   return p.bytes;
@@ -912,9 +918,9 @@ int aios_linear_rows_ws(const void* x, int64_t x_stride, const void* weight, int
   a.N = out_features;
   const bool silu = epilogue == AIOS_EPILOGUE_SILU_MUL;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (rows_form(rows, out_features, in_features, silu, device_cus()) &&
+  const bool ws = workspace && ((uintptr_t)workspace & 15) == 0;
+  if (rows_form(rows, out_features, in_features, silu, ws, device_cus()) &&
       aios::rows_gemm_fits(a, silu)) {
-    const bool ws = workspace && ((uintptr_t)workspace & 15) == 0;
     aios::RowsPlan p;
     bool ok = aios::rows_gemm_plan(rows, out_features, in_features, silu, ws, device_cus(), &p);
     if (ok && p.bytes > workspace_bytes)
