@@ -150,6 +150,8 @@ def _attention_step_us(eng, reps: int = 30) -> float:
     as they do between the projections of the full step."""
     import torch
 
+    from aios_amd.core import captured
+
     g = next(reversed(eng._graphs.values()))
     rt = eng.rt
     c = rt.config
@@ -171,7 +173,7 @@ def _attention_step_us(eng, reps: int = 30) -> float:
     with torch.inference_mode():
         with torch.cuda.stream(s):
             body()
-        with torch.cuda.graph(graph, stream=s):
+        with captured(graph, s):
             body()
     e0 = torch.cuda.Event(enable_timing=True)
     e1 = torch.cuda.Event(enable_timing=True)
@@ -599,6 +601,7 @@ def attnres_pipeline(seed: int, warmups: int = 5, iters: int = 50) -> dict:
 
     import torch
 
+    from aios_amd.core import captured
     from aios_amd.layers import HipOps
     from aios_amd.minimind_ime import DepthBank
 
@@ -654,7 +657,7 @@ def attnres_pipeline(seed: int, warmups: int = 5, iters: int = 50) -> dict:
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(s):
         run()
-        with torch.cuda.graph(graph, stream=s):
+        with captured(graph, s):
             out = run()
     torch.cuda.current_stream(dev).wait_stream(s)
     graph_ms = []
@@ -769,6 +772,7 @@ def main() -> int:
     import torch
 
     from aios_amd import paged
+    from aios_amd.core import captured
     from aios_amd.kernel import store_cache
     from aios_amd.workloads import SHAPES, decode_bytes_per_layer, kv_append_bytes, make_decode_workload
 
@@ -826,7 +830,7 @@ def main() -> int:
     torch.cuda.synchronize()
     eager_out = out.clone()
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph, stream=s):
+    with captured(graph, s):
         step()
     with torch.cuda.stream(s):
         for _ in range(args.warmup):
