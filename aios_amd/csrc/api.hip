@@ -99,7 +99,7 @@ bool rows_form(int64_t rows, int64_t n, int64_t k, bool silu, bool workspace, in
   if (silu)
     return 4 * tiles <= cus || !((2 * tiles <= cus && k <= 1792) || (4 * tiles <= 3 * cus && k <= 1280));
   if (tiles > cus) return rows > 2 || (k > 1280 && (k < 3072 || k > 4096));
-  if (k <= 1792 || (8 * tiles > 7 * cus && k <= 4608)) return false;
+  if (k <= 1792 || (8 * tiles > 7 * cus && (k < 4096 || (k <= 4608 && rows <= 12)))) return false;
   if (k <= 2688) return 2 * tiles > cus || (k > 2304 && rows > 12 && workspace);
   return k > 4608 || rows > 8 || n < (rows <= 4 && k <= 4096 ? 1024 : 2048);
 }
